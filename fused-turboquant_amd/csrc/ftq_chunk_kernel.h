@@ -1,0 +1,470 @@
+// Attention of a chunk of consecutive query tokens of one sequence over a
+// compressed K/V cache (the continuation of a chunked prefill): causal, every
+// query row r attends positions [lo(r), past + r + 1).
+//
+// The decode kernels dequantise the cache once per (query token, kv head); a
+// chunk of n tokens that goes through them as n synthetic sequences
+// dequantises it n times.  Here the cache is dequantised once per chunk, into
+// the exact operands of the matrix cores (not into rounded K and V), and a
+// flash-attention kernel then shares every 64-token tile among 128 (64 at
+// D = 256) query columns:
+//   gather   codes -> K table values (f16, or f16 hi + lo where the decode
+//            kernel of that format keeps fp32 products) and V codes (centred,
+//            exact in f16), in MFMA fragment order, plus 4 floats per token:
+//            K factor, bias (0, or -inf for a position without a page), V
+//            factor, V minimum
+//   queries  rotated, scaled by scale * log2 e, f16 hi + lo, fragment order
+//   attend   S^T = K Q^T, softmax in the log2 domain, O^T = V^T P^T
+//
+// Fragment order: lane (m, g) of v_mfma_f32_16x16x32_f16 (m = lane & 15,
+// g = lane >> 4) reads 16 contiguous bytes, and a wave 1 KB:
+//   K  [16-token tile][32-dim step s][part][lane]: token m, dims 32 s + 8 g + j
+//   V  [32-token tile][16-dim block b][lane]: dim 16 b + m, tokens 4 g + j and
+//      16 + 4 g + j (j < 4) -- the row order of the S^T accumulators, so P goes
+//      from the score registers into the P.V operand without a shuffle
+//   Q  [16-column tile][s][part][lane]: column m, dims 32 s + 8 g + j
+// A column is a (query row, head of the kv head's group) pair, row-major.
+#pragma once
+
+#include "ftq_attn_dev.h"
+#include "ftq_merge.h"
+#include "ftq_v1_dev.h"
+
+namespace ftq {
+
+// Query columns of a workgroup (4 waves) and tokens of a tile.
+template <int D, bool KHL> struct ChunkGeo {
+  static constexpr int CT = D == 256 ? 1 : 2;     // 16-column tiles per wave
+  static constexpr int COLS = 64 * CT;
+  static constexpr int TK = D == 64 ? 64 : 32;
+  static constexpr int NS = D / 32, NB = D / 16, NT = TK / 16, NP = TK / 32;
+};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+struct ChunkAttn {
+  const u32x4 *kf, *vf, *qf;   // fragments: [kv head][...]
+  const float* tok;            // [kv head][tile][4][TK]: K factor, bias, V factor, V minimum
+  const float* qfac;           // per column factor of the scores ([kv head][column]); KHL only
+  int64_t kstride, vstride, qstride;  // uint4 per kv head
+  int64_t tstride;             // floats per kv head
+  int cstride;                 // columns per kv head (qfac)
+  int nq, G, hq, hkv, past, window;
+  int seg0, seg1;              // token range held by the fragments (seg0 a multiple of 64)
+  int splits, split0, splits_all;  // splits of this launch, its first split, all splits of the row
+  float *wo, *wl;              // partial outputs / log-sum-exps, or
+  void* out;                   // the output itself (wo == null)
+  int ot, rot;                 // output dtype; MergeRot of the direct output (ROT_NONE / PLAIN / SIGNS)
+  const float* signs;
+  float oscale;                // V fragments' common scale, and of the un-rotation (direct output only)
+  int64_t o_row, o_head;       // output strides (elements) of a query row and of a head
+};
+
+// x of the lane 16 (32) lanes up or down: the butterfly pair of lane bit 4 (5)
+__device__ __forceinline__ float fwht_pair16(float x, bool upper) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+  return upper ? a - b : a + b;
+}
+__device__ __forceinline__ float fwht_pair32(float x, bool upper) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+  return upper ? a - b : a + b;
+}
+
+// f16 pair of two floats, each rounded to nearest (v_cvt_pk_f16_f32)
+__device__ __forceinline__ uint32_t pk_f16(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), half2_t));
+}
+// x - f16 half of w
+__device__ __forceinline__ float f16_rest(float x, uint32_t w, int half) {
+  return x - (float)__builtin_bit_cast(half2_t, w)[half];
+}
+
+// D: head dim; NH: f16 parts of the query and of the weights (2: ~22 bits, as
+// the v1 decode kernels; 1: f16); KHL: K fragments as hi + lo and the query
+// scaled per column (formats whose decode runs fp32 products); ZM: V has a
+// per-token minimum, and positions may lack a page.
+template <int D, int NH, bool KHL, bool ZM>
+__global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
+  using C = ChunkGeo<D, KHL>;
+  constexpr int CT = C::CT, TK = C::TK, NS = C::NS, NB = C::NB, NT = C::NT, NP = C::NP;
+  constexpr int KP = KHL ? 2 : 1;
+  constexpr int KU = NT * NS * KP * 64, VU = NP * NB * 64;  // 16-byte units of a tile
+  constexpr int KT = KU / 256 / KP, VT = VU / 256;
+  __shared__ u32x4 kb[2][KU];
+  __shared__ u32x4 vb[2][VU];
+  __shared__ __attribute__((aligned(16))) float tb[2][4][TK];
+
+  // kv head fastest: with 8 kv heads each XCD (workgroups are dealt to the 8
+  // XCDs in turn) reads one head's fragments, which then stay in its L2
+  const int kvh = blockIdx.x % a.hkv;
+  const int blk = (int)(gridDim.x / a.hkv) - 1 - (int)(blockIdx.x / a.hkv);  // longest rows first
+  const int split = blockIdx.y;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int n = lane & 15, g = lane >> 4;
+  const int ncols = a.nq * a.G;
+
+  // the rows of this workgroup, wave and lane
+  const int c0 = blk * C::COLS;
+  const int r_lo = c0 / a.G, r_hi = (min(c0 + C::COLS, ncols) - 1) / a.G;
+  const int wc0 = c0 + wave * 16 * CT;
+  const int wr_lo = min(wc0 / a.G, a.nq - 1), wr_hi = min((wc0 + 16 * CT - 1) / a.G, a.nq - 1);
+  const int first = a.window > 0 ? max(0, a.past + r_lo + 1 - a.window) : 0;
+  const int t0 = max(first, a.seg0) / TK;
+  const int t1 = (min(a.past + r_hi + 1, a.seg1) + TK - 1) / TK;
+  const int nt = t1 > t0 ? t1 - t0 : 0;
+  const int per = (nt + a.splits - 1) / a.splits;
+  const int tb0 = t0 + split * per, tb1 = min(tb0 + per, t1);
+  // positions every / any row of the wave attends
+  const int w_all = a.past + wr_lo + 1;                                     // below: in every row's causal range
+  const int w_from = a.window > 0 ? max(0, a.past + wr_hi + 1 - a.window) : 0;  // from: in every row's window
+  int lim[CT], lo[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    const int r = min((wc0 + 16 * ct + n) / a.G, a.nq - 1);
+    lim[ct] = a.past + r + 1;
+    lo[ct] = a.window > 0 ? max(0, lim[ct] - a.window) : 0;
+  }
+
+  const u32x4* kf = a.kf + (int64_t)kvh * a.kstride;
+  const u32x4* vf = a.vf + (int64_t)kvh * a.vstride;
+  const float* tk = a.tok + (int64_t)kvh * a.tstride;
+  const int tseg = a.seg0 / TK;
+  u32x4 rk[KT], rl[KHL ? KT : 1], rv[VT];
+  float rt = 0.f;
+  auto fetch = [&](int t) __attribute__((always_inline)) {
+    const u32x4* pk = kf + (int64_t)(t - tseg) * KU + tid;
+    const u32x4* pv = vf + (int64_t)(t - tseg) * VU + tid;
+#pragma unroll
+    for (int j = 0; j < KT; ++j) rk[j] = pk[256 * j];
+    if constexpr (KHL) {
+#pragma unroll
+      for (int j = 0; j < KT; ++j) rl[j] = pk[256 * (KT + j)];
+    }
+#pragma unroll
+    for (int j = 0; j < VT; ++j) rv[j] = pv[256 * j];
+    if (tid < 4 * TK) rt = tk[(int64_t)(t - tseg) * 4 * TK + tid];
+  };
+  auto commit = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < KT; ++j) kb[p][tid + 256 * j] = rk[j];
+    if constexpr (KHL) {
+#pragma unroll
+      for (int j = 0; j < KT; ++j) kb[p][tid + 256 * (KT + j)] = rl[j];
+    }
+#pragma unroll
+    for (int j = 0; j < VT; ++j) vb[p][tid + 256 * j] = rv[j];
+    if (tid < 4 * TK) (&tb[p][0][0])[tid] = rt;
+  };
+
+  if (tb0 < tb1) fetch(tb0);
+  // the query operands of the wave's columns
+  half8 qh[CT][NS], ql[NH == 2 ? CT : 1][NH == 2 ? NS : 1];
+  float qs[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    const u32x4* pq = a.qf + (int64_t)kvh * a.qstride + (int64_t)(wc0 / 16 + ct) * (NS * NH * 64) + lane;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      qh[ct][s] = __builtin_bit_cast(half8, pq[(s * NH) * 64]);
+      if constexpr (NH == 2) ql[ct][s] = __builtin_bit_cast(half8, pq[(s * NH + 1) * 64]);
+    }
+    qs[ct] = KHL ? a.qfac[(int64_t)kvh * a.cstride + wc0 + 16 * ct + n] : 1.f;
+  }
+
+  constexpr float TAU = 8.f;        // weights stay below 2^TAU
+  constexpr float MINF = -3.0e38f;  // running maximum of a column with no position yet
+  float m_run[CT], l_run[CT], z_run[CT];
+  floatx4 acc[CT][NB];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    m_run[ct] = MINF;
+    l_run[ct] = z_run[ct] = 0.f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[ct][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  auto process = [&](int t, int p) __attribute__((always_inline)) {
+    floatx4 s[NT][CT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) s[k][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 sl[KHL ? NT : 1][KHL ? CT : 1];  // the low parts' products, summed apart
+    if constexpr (KHL) {
+#pragma unroll
+      for (int k = 0; k < NT; ++k)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) sl[k][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int d = 0; d < NS; ++d)
+#pragma unroll
+      for (int k = 0; k < NT; ++k) {
+        half8 x = __builtin_bit_cast(half8, kb[p][((k * NS + d) * KP) * 64 + lane]);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, qh[ct][d], s[k][ct], 0, 0, 0);
+          if constexpr (KHL) sl[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, ql[ct][d], sl[k][ct], 0, 0, 0);
+          else if constexpr (NH == 2) s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, ql[ct][d], s[k][ct], 0, 0, 0);
+        }
+        if constexpr (KHL) {
+          x = __builtin_bit_cast(half8, kb[p][((k * NS + d) * KP + 1) * 64 + lane]);
+  #pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+            sl[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, qh[ct][d], sl[k][ct], 0, 0, 0);
+        }
+      }
+    const bool edge = t * TK + TK > w_all || t * TK < w_from;  // wave-uniform
+    // scores: x K factor (and the column's), + bias; masked on the edges
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+      const float4 f4 = *reinterpret_cast<const float4*>(&tb[p][0][16 * k + 4 * g]);
+      const float fa[4] = {f4.x, f4.y, f4.z, f4.w};
+      float ba[4] = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (ZM) {
+        const float4 b4 = *reinterpret_cast<const float4*>(&tb[p][1][16 * k + 4 * g]);
+        ba[0] = b4.x; ba[1] = b4.y; ba[2] = b4.z; ba[3] = b4.w;
+      }
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float y = s[k][ct][i];
+          if constexpr (KHL) y = (y + sl[k][ct][i]) * qs[ct];
+          s[k][ct][i] = ZM ? __builtin_fmaf(y, fa[i], ba[i]) : y * fa[i];
+        }
+    }
+    if (edge) {
+#pragma unroll
+      for (int k = 0; k < NT; ++k)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int pos = t * TK + 16 * k + 4 * g + i;
+            if (pos >= lim[ct] || pos < lo[ct]) s[k][ct][i] = -INFINITY;
+          }
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      float tm = s[0][ct][0];
+#pragma unroll
+      for (int k = 0; k < NT; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tm = fmaxf(tm, s[k][ct][i]);
+      tm = warp_max_q(tm);
+      if (__builtin_amdgcn_ballot_w64(tm > m_run[ct] + TAU) != 0) {  // wave-uniform, rare
+        const float mn = fmaxf(m_run[ct], tm);
+        const float al = __builtin_amdgcn_exp2f(m_run[ct] - mn);
+        m_run[ct] = mn;
+        l_run[ct] *= al;
+        z_run[ct] *= al;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[ct][b] *= al;
+      }
+    }
+    // weights: p, p x V minimum kept aside, p x V factor as f16 parts
+    u32x4 ph[NP][CT], pl[NH == 2 ? NP : 1][NH == 2 ? CT : 1];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+      const float4 v4 = *reinterpret_cast<const float4*>(&tb[p][2][16 * k + 4 * g]);
+      const float va[4] = {v4.x, v4.y, v4.z, v4.w};
+      float za[4] = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (ZM) {
+        const float4 z4 = *reinterpret_cast<const float4*>(&tb[p][3][16 * k + 4 * g]);
+        za[0] = z4.x; za[1] = z4.y; za[2] = z4.z; za[3] = z4.w;
+      }
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        float w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = __builtin_amdgcn_exp2f(s[k][ct][i] - m_run[ct]);
+          l_run[ct] += e;
+          float vv = va[i], zz = za[i];
+          if (edge) {  // a hidden position's factors may be infinite or NaN
+            const bool hid = s[k][ct][i] == -INFINITY;
+            vv = hid ? 0.f : vv;
+            zz = hid ? 0.f : zz;
+          }
+          if constexpr (ZM) z_run[ct] = __builtin_fmaf(e, zz, z_run[ct]);
+          w[i] = e * vv;
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t hi = pk_f16(w[2 * h], w[2 * h + 1]);
+          ph[k >> 1][ct][2 * (k & 1) + h] = hi;
+          if constexpr (NH == 2)
+            pl[k >> 1][ct][2 * (k & 1) + h] = pk_f16(f16_rest(w[2 * h], hi, 0), f16_rest(w[2 * h + 1], hi, 1));
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const half8 x = __builtin_bit_cast(half8, vb[p][(k * NB + b) * 64 + lane]);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8, ph[k][ct]), acc[ct][b], 0, 0, 0);
+          if constexpr (NH == 2)
+            acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8, pl[k][ct]), acc[ct][b], 0, 0, 0);
+        }
+      }
+  };
+
+  // one barrier a tile: a buffer is refilled in the iteration after its
+  // readers passed the barrier that ended theirs
+  if (tb0 < tb1) commit(0);
+  // the query operands have arrived before the loop (vmcnt 0), or the loop
+  // would wait for them behind each next tile's loads
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+  int p = 0;
+  for (int t = tb0; t < tb1; ++t, p ^= 1) {
+    if (t + 1 < tb1) fetch(t + 1);
+    process(t, p);
+    if (t + 1 < tb1) commit(p ^ 1);
+    __syncthreads();
+  }
+
+  // ---- output: lane (n, g) holds dims 16 b + 4 g + i of column n ----
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    const float L = warp_sum_q(l_run[ct]);
+    const float Z = ZM ? warp_sum_q(z_run[ct]) : 0.f;
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    float y[NB][4];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[b][i] = L > 0.f ? (acc[ct][b][i] + Z) * inv : 0.f;
+    const int col = wc0 + 16 * ct + n;
+    const bool live = col < ncols;
+    const int r = live ? col / a.G : 0, h = kvh * a.G + (live ? col - r * a.G : 0);
+    if (a.wo != nullptr) {
+      const int64_t row = ((int64_t)r * a.hq + h) * a.splits_all + a.split0 + split;
+      if (live) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          *reinterpret_cast<float4*>(a.wo + row * D + 16 * b + 4 * g) = make_float4(y[b][0], y[b][1], y[b][2], y[b][3]);
+        if (g == 0) a.wl[row] = L > 0.f ? m_run[ct] + __builtin_log2f(L) : -INFINITY;
+      }
+      continue;
+    }
+    if (a.rot != ROT_NONE) {  // H o: dim bits 0-1 and 4.. in registers, bits 2-3 across the lane rows
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const float u0 = y[b][0] + y[b][1], u1 = y[b][0] - y[b][1], u2 = y[b][2] + y[b][3], u3 = y[b][2] - y[b][3];
+        y[b][0] = u0 + u2; y[b][1] = u1 + u3; y[b][2] = u0 - u2; y[b][3] = u1 - u3;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[b][i] = fwht_pair32(fwht_pair16(y[b][i], g & 1), g & 2);
+      }
+#pragma unroll
+      for (int st = 1; st < NB; st <<= 1)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          if ((b & st) == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float u = y[b][i], v = y[b + st][i];
+              y[b][i] = u + v;
+              y[b + st][i] = u - v;
+            }
+          }
+    }
+    if (live) {
+      const int64_t off = (int64_t)r * a.o_row + (int64_t)h * a.o_head;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o[i] = y[b][i] * a.oscale;
+          if (a.rot == ROT_SIGNS) o[i] *= a.signs[16 * b + 4 * g + i];
+        }
+        if (a.ot == F32) store_small<F32, 4>(a.out, off + 16 * b + 4 * g, o);
+        else if (a.ot == F16) store_small<F16, 4>(a.out, off + 16 * b + 4 * g, o);
+        else store_small<BF16, 4>(a.out, off + 16 * b + 4 * g, o);
+      }
+    }
+  }
+}
+
+// Queries of a chunk: E = D / 16 elements per lane of a 16-lane group, rotated
+// (H, or x M), times qscale, to fragments of NH f16 parts.  KHL: each query is
+// first scaled by the power of two that puts its largest magnitude in
+// [256, 512), so that the low parts of the others stay normal f16 numbers;
+// qfac takes the inverse.
+template <int D, int QT, int NH, bool KHL>
+__global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict__ query, int64_t q_row, int64_t q_head,
+                                                          int nq, int hq, int hkv, const float* __restrict__ signs,
+                                                          const float* __restrict__ rot, int rotate, float qscale,
+                                                          uint2* __restrict__ qf, int64_t qstride2,
+                                                          float* __restrict__ qfac, int cstride) {
+  constexpr int E = D / 16, NS = D / 32;
+  __shared__ float rows[16][D + 4];
+  const int grp = threadIdx.x >> 4, l16 = threadIdx.x & 15;
+  const int64_t v = (int64_t)blockIdx.x * 16 + grp;
+  const bool live = v < (int64_t)nq * hq;
+  const int r = live ? (int)(v / hq) : 0, head = live ? (int)(v - (int64_t)r * hq) : 0;
+  const int G = hq / hkv, kvh = head / G, col = r * G + head - kvh * G;
+  float y[E];
+  load_elems<QT, E>(query, (int64_t)r * q_row + (int64_t)head * q_head + l16 * E, y);
+  if (signs != nullptr) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) y[i] *= signs[l16 * E + i];
+  }
+  if (rot != nullptr) rot_matrix_lanes<D, E>(y, rot, rows[grp], l16);
+  else if (rotate) fwht_lanes<E, 16>(y, l16);
+  float up = 1.f;
+  if constexpr (KHL) {
+    float mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      y[i] *= qscale;
+      mx = fmaxf(mx, fabsf(y[i]));
+    }
+    mx = fmaxf(mx, lane_xor<1>(mx));
+    mx = fmaxf(mx, lane_xor<2>(mx));
+    mx = fmaxf(mx, lane_xor<4>(mx));
+    mx = fmaxf(mx, lane_xor<8>(mx));
+    const int e = (int)((__float_as_uint(mx) >> 23) & 255u);  // mx in [2^(e-127), 2^(e-126))
+    const int ue = min(max(135 + 127 - e, 1), 253);           // 2^(8 - (e - 127)), kept normal both ways
+    up = __uint_as_float((uint32_t)ue << 23);
+    if (live && l16 == 0) qfac[(int64_t)kvh * cstride + col] = __uint_as_float((uint32_t)(254 - ue) << 23);
+  } else {
+    up = qscale;
+  }
+  if (!live) return;
+#pragma unroll
+  for (int i = 0; i < E; i += 4) {
+    float x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = y[i + j] * up;
+    const int dim = l16 * E + i, s = dim >> 5, gg = (dim >> 3) & 3, half = (dim >> 2) & 1;
+    uint2* dst = qf + (int64_t)kvh * qstride2 + ((int64_t)(col >> 4) * (NS * NH * 64) + (s * NH) * 64 + gg * 16 + (col & 15)) * 2 + half;
+    const uint32_t h0 = pk_f16(x[0], x[1]), h1 = pk_f16(x[2], x[3]);
+    dst[0] = make_uint2(h0, h1);
+    if constexpr (NH == 2)
+      dst[128] = make_uint2(pk_f16(f16_rest(x[0], h0, 0), f16_rest(x[1], h0, 1)),
+                            pk_f16(f16_rest(x[2], h1, 0), f16_rest(x[3], h1, 1)));
+  }
+}
+
+template <int D, int NH, bool KHL>
+hipError_t launch_chunk_query(const void* query, int qt, int64_t q_row, int64_t q_head, int nq, int hq, int hkv,
+                              const float* signs, const float* rot, int rotate, float qscale, uint4* qf,
+                              int64_t qstride, float* qfac, int cstride, hipStream_t st) {
+  const dim3 grid((unsigned)(((int64_t)nq * hq + 15) / 16)), block(256);
+  uint2* q2 = reinterpret_cast<uint2*>(qf);
+  if (qt == F32) chunk_query_kernel<D, F32, NH, KHL><<<grid, block, 0, st>>>(query, q_row, q_head, nq, hq, hkv, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
+  else if (qt == F16) chunk_query_kernel<D, F16, NH, KHL><<<grid, block, 0, st>>>(query, q_row, q_head, nq, hq, hkv, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
+  else chunk_query_kernel<D, BF16, NH, KHL><<<grid, block, 0, st>>>(query, q_row, q_head, nq, hq, hkv, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
+  return hipGetLastError();
+}
+
+}  // namespace ftq

@@ -241,6 +241,43 @@ void v1_decode_attention(const at::Tensor& query, const at::Tensor& kv_cache, co
       rotation.has_value() ? rotation->data_ptr<float>() : nullptr, stream_of(query)));
 }
 
+// Causal attention of the last query.size(0) of past_len + query.size(0)
+// stored positions of one sequence; the dequantised fragments and split
+// partials live in a workspace from torch's caching allocator (as large as
+// the chunk and its context need, returned to the stream's pool afterwards).
+void v1_chunk_attention(const at::Tensor& query, const at::Tensor& kv_cache, const at::Tensor& block_row,
+                        int64_t past_len, const std::optional<at::Tensor>& centroids, int64_t key_bits,
+                        int64_t value_bits, double scale, int64_t v_flags, int64_t window, at::Tensor& out,
+                        const std::optional<at::Tensor>& rotation) {
+  contig(query, "query");
+  on_device(kv_cache, "kv_cache");
+  contig(block_row, "block_row");
+  contig(out, "out");
+  TORCH_CHECK(query.dim() == 3 && out.sizes() == query.sizes(), "fused_tq: query and out must be [n, Hq, d]");
+  TORCH_CHECK(kv_cache.dim() == 4 && kv_cache.scalar_type() == at::kByte && kv_cache.stride(3) == 1,
+              "fused_tq: kv_cache must be uint8 [num_blocks, block_size, Hkv, slot] with contiguous slots");
+  TORCH_CHECK(block_row.scalar_type() == at::kInt, "fused_tq: block_row must be int32");
+  TORCH_CHECK_VALUE(past_len >= 0 && past_len <= INT32_MAX && window >= 0 && window <= INT32_MAX &&
+                        query.size(0) <= INT32_MAX && block_row.numel() <= INT32_MAX,
+                    "fused_tq: past_len / window / token counts out of range");
+  if (centroids.has_value()) contig(*centroids, "centroids");
+  if (rotation.has_value()) contig(*rotation, "rotation");
+  const c10::DeviceGuard g(query.device());
+  const int n = (int)query.size(0), hq = (int)query.size(1), d = (int)query.size(2), hkv = (int)kv_cache.size(2);
+  if (n == 0) return;
+  const int64_t need = ftq_v1_chunk_workspace_bytes(n, hq, hkv, d, (int)past_len, (int)key_bits, (int)value_bits,
+                                                    (int)v_flags, (int)window);
+  TORCH_CHECK_VALUE(need >= 0, "fused_tq: chunk attention does not take this head_dim, code width or token count");
+  at::Tensor ws = at::empty({need}, query.options().dtype(at::kByte));
+  check_rc(ftq_v1_chunk_attention(
+      query.data_ptr(), dt(query), kv_cache.data_ptr<uint8_t>(), kv_cache.size(0), (int)kv_cache.size(1),
+      kv_cache.stride(0), kv_cache.stride(1), kv_cache.stride(2), block_row.data_ptr<int32_t>(),
+      (int)block_row.numel(), (int)past_len, n, hq, hkv, d,
+      centroids.has_value() ? centroids->data_ptr<float>() : nullptr, (int)key_bits, (int)value_bits, (float)scale,
+      (int)v_flags, (int)window, ws.data_ptr(), need, out.data_ptr(), dt(out),
+      rotation.has_value() ? rotation->data_ptr<float>() : nullptr, stream_of(query)));
+}
+
 // ---- raw fp16 slots (boundary layers) -------------------------------------
 
 void raw_store(const at::Tensor& key, const at::Tensor& value, at::Tensor& kv_cache, const at::Tensor& slot_mapping) {
@@ -301,6 +338,8 @@ TORCH_LIBRARY(fused_tq, m) {
   m.def("v1_decode_attention(Tensor query, Tensor kv_cache, Tensor block_table, Tensor seq_lens, "
         "Tensor? kv_start, Tensor centroids, int key_bits, int value_bits, float scale, int v_flags, "
         "int num_splits, Tensor(a!) workspace, Tensor(b!) out, Tensor(c!)? lse, Tensor? rotation) -> ()");
+  m.def("v1_chunk_attention(Tensor query, Tensor kv_cache, Tensor block_row, int past_len, Tensor? centroids, "
+        "int key_bits, int value_bits, float scale, int v_flags, int window, Tensor(a!) out, Tensor? rotation) -> ()");
   m.def("raw_store(Tensor key, Tensor value, Tensor(a!) kv_cache, Tensor slot_mapping) -> ()");
   m.def("raw_decode_attention(Tensor query, Tensor kv_cache, Tensor block_table, Tensor seq_lens, "
         "Tensor? kv_start, float scale, int num_splits, Tensor(a!) workspace, Tensor(b!) out, "
@@ -316,6 +355,7 @@ TORCH_LIBRARY_IMPL(fused_tq, CUDA, m) {
   m.impl("paged_decode_attention", &paged_decode_attention);
   m.impl("v1_store", &v1_store);
   m.impl("v1_decode_attention", &v1_decode_attention);
+  m.impl("v1_chunk_attention", &v1_chunk_attention);
   m.impl("raw_store", &raw_store);
   m.impl("raw_decode_attention", &raw_decode_attention);
 }

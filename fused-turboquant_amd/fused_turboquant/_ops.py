@@ -50,8 +50,8 @@ def _register_fakes() -> None:
         return x.new_empty(x.shape, dtype=out_dtype)
 
     # operators that only write their (a!) arguments
-    for name in ("paged_store", "paged_decode_attention", "v1_store", "v1_decode_attention", "raw_store",
-                 "raw_decode_attention"):
+    for name in ("paged_store", "paged_decode_attention", "v1_store", "v1_decode_attention",
+                 "v1_chunk_attention", "raw_store", "raw_decode_attention"):
         torch.library.register_fake(lib + name)(lambda *args, **kwargs: None)
 
 

@@ -444,6 +444,38 @@ def v1_decode_attention(query: torch.Tensor, kv_cache: torch.Tensor, block_table
     return out
 
 
+RAW_BITS = 16  # key_bits = value_bits of raw fp16 slots in ``v1_chunk_attention``
+
+
+def v1_chunk_attention(query: torch.Tensor, kv_cache: torch.Tensor, block_row: torch.Tensor, past_len: int,
+                       centroids: torch.Tensor | None, key_bits: int, value_bits: int, scale: float,
+                       v_rotate: bool = False, window: int | None = None, out: torch.Tensor | None = None,
+                       rotation: torch.Tensor | None = None, key_fp8: bool = False) -> torch.Tensor:
+    """Attention of the last n of ``past_len + n`` stored positions of one
+    sequence, query [n, Hq, d] -> [n, Hq, d]: row i attends positions
+    [max(0, past_len + i + 1 - window), past_len + i + 1) of the slots that
+    ``block_row`` (int32) maps.  ``centroids`` sorted float32 (None for fp8
+    keys and for raw slots, ``key_bits = value_bits = RAW_BITS``).  Uniform V
+    codes only: Lloyd-Max V goes through ``v1_decode_attention``."""
+    n, hq, d = query.shape
+    if key_bits != RAW_BITS:
+        _check_bits(d, key_bits, value_bits, key_fp8)
+    if block_row.dtype != torch.int32 or block_row.dim() != 1:
+        raise ValueError("block_row must be int32 [max_blocks]")
+    tensors = [query, kv_cache, block_row] + ([centroids] if centroids is not None else [])
+    dev = _lib.require_device(*tensors)
+    q = query.contiguous()
+    if q.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        q = q.float()
+    if out is None:
+        out = torch.empty(n, hq, d, dtype=q.dtype, device=dev)
+    _strides(kv_cache)
+    rot = _rotation_arg(rotation, d, dev) if rotation is not None else None
+    _ops.ops().v1_chunk_attention(q, kv_cache, block_row.contiguous(), int(past_len), centroids, key_bits, value_bits,
+                                  float(scale), _v_flags(v_rotate, False, key_fp8), int(window or 0), out, rot)
+    return out
+
+
 class TurboQuantV1Layer:
     """Per-layer state of the v1 backend for ``kind=rht``: sorted centroids and
     midpoints (reference ``rotation/matrix.py:34-42``), bit widths and the

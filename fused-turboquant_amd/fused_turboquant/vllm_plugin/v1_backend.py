@@ -20,10 +20,10 @@ Per call:
   batch, grouped K/V (``enable_gqa``, ``:1355-1358``), one launch per run of
   consecutive fresh sequences of one length (the reference uses flash-attn
   varlen there, ``:1283-1443``).
-* prefill continuing a cached sequence -> the decode kernel with one
-  synthetic sequence per query token (seq_len = cached + i + 1, same block
-  table row): causal attention over the stored slots, the reference's
-  continuation path (``:1359-1384``).
+* prefill continuing a cached sequence -> the chunk kernel, causal attention
+  of the new tokens over the stored slots (the reference's continuation path,
+  ``:1359-1384``, runs its decode kernel over one synthetic sequence per query
+  token, as is done here for a few tokens).
 
 Boundary-protection layers (a plain cache dtype such as ``"auto"``; reference
 ``:335-366``) follow ``TURBOQUANT_BOUNDARY_PROTECT``: ``fp16`` stores raw fp16
@@ -476,7 +476,7 @@ class FusedTurboQuantV1Impl(_ImplBase):
         """Prefill sequences nd.. of the batch (tokens ndt..N).  A run of
         consecutive fresh sequences of one length is one batched SDPA over
         views of q / k / v (no copies, grouped K/V); a continuing sequence
-        runs the decode kernel with one synthetic row per query token."""
+        attends its stored slots."""
         qsl = md.query_start_loc.tolist()
         sls = md.seq_lens.tolist()
         N = q.shape[0]
@@ -505,12 +505,29 @@ class FusedTurboQuantV1Impl(_ImplBase):
                                                                                    self.head_size)
                 i = j
             else:
-                # continuation: one synthetic decode per query token over the stored slots
-                row = md.block_table[i:i + 1].to(torch.int32).expand(n_q, -1).contiguous()
-                syn = torch.arange(past + 1, past + n_q + 1, device=q.device, dtype=torch.int32)
-                out[a - ndt:b - ndt] = self._decode(q[a:b], kv_cache, row, syn, st, max_seq_len=sls[i])
+                self._continue(q[a:b], kv_cache, md.block_table[i], past, st, out[a - ndt:b - ndt])
                 i += 1
         return out
+
+    def _continue(self, q, kv_cache, block_row, past: int, st, out) -> None:
+        """The next n tokens of a cached sequence over their stored slots: the
+        chunk kernel (the cache dequantised once), or, for a few tokens and
+        for Lloyd-Max V, the decode kernel over one synthetic sequence per
+        query token."""
+        n_q = q.shape[0]
+        row = block_row.to(torch.int32)
+        raw = self._is_raw
+        matrix = self.head_size == 128 and (raw or (2 <= self.key_bits <= 4 and 2 <= self.value_bits <= 4))
+        enough = n_q >= (_CHUNK_MIN_TOKENS if matrix else _CHUNK_MIN_TOKENS_VALU)
+        if enough and not (self.v_lloyd_max and self.value_bits == 4):
+            V1.v1_chunk_attention(q, kv_cache, row, past, None if raw or self.key_fp8 else st.centroids, self.key_bits,
+                                  self.value_bits, self.scale, v_rotate=not raw and st.v_rotate,
+                                  window=self.sliding_window, out=out, rotation=None if raw else st.rotation,
+                                  key_fp8=self.key_fp8)
+            return
+        rows = row[None].expand(n_q, -1).contiguous()
+        syn = torch.arange(past + 1, past + n_q + 1, device=q.device, dtype=torch.int32)
+        out.copy_(self._decode(q, kv_cache, rows, syn, st, max_seq_len=past + n_q))
 
     def _fresh_attention(self, q, k, v):
         """Causal attention of fresh sequences, q [G, L, Hq, D] and k / v
@@ -537,6 +554,13 @@ class FusedTurboQuantV1Impl(_ImplBase):
 # windowed one (its mask is block x (block + window) booleans)
 _FRESH_BATCH_TOKENS = 32768
 _WINDOW_QUERY_BLOCK = 2048
+# Query tokens of a continuing sequence from which the chunk kernel runs.  It
+# pays one pass over the context whatever the chunk; the decode kernel pays one
+# per token.  Measured (bf16, K4V4, 8 kv heads, group 4; decode / chunk us):
+# d = 128, 8 tokens over 30000 positions 79 / 119, 16 tokens 132 / 118, over
+# 5120 44 / 44; d = 64, 4 tokens 85 / 91, 8 tokens 132 / 90.
+_CHUNK_MIN_TOKENS = 16
+_CHUNK_MIN_TOKENS_VALU = 8  # formats whose decode runs on the VALU
 _GQA_KERNELS: Optional[bool] = None  # whether torch's fused SDPA kernels take grouped K/V here
 
 

@@ -387,6 +387,28 @@ int ftq_v1_decode_attention_noalloc(const void* query, int q_dtype, const uint8_
 int64_t ftq_raw_slot_bytes(int d);
 
 /*
+ * Attention of a chunk: the last n_query of past_len + n_query positions of
+ * one sequence, all of them already stored, each query row attending the
+ * positions up to its own (and, with window > 0, its last `window`).  The
+ * continuation of a chunked prefill (reference vllm_plugin/v1_backend.py:
+ * 1359-1384); the same result as ftq_v1_decode_attention over one synthetic
+ * sequence per query token, with the cache dequantised once per chunk.
+ *   query, out [n_query, num_q_heads, d]; block_row [max_blocks] int32
+ *   key_bits, value_bits: as ftq_v1_decode_attention, or both 16 for raw fp16
+ *   slots (v_flags 0, no rotation, centroids unused); v_flags: FTQ_V1 bits 0
+ *   (un-rotate V) and 2 (fp8 keys)
+ *   workspace: ftq_v1_chunk_workspace_bytes (-1: arguments out of range)
+ */
+int64_t ftq_v1_chunk_workspace_bytes(int n_query, int num_q_heads, int num_kv_heads, int d, int past_len,
+                                     int key_bits, int value_bits, int v_flags, int window);
+int ftq_v1_chunk_attention(const void* query, int q_dtype, const uint8_t* kv_cache, int64_t num_blocks,
+                           int block_size, int64_t stride_block, int64_t stride_pos, int64_t stride_head,
+                           const int32_t* block_row, int max_blocks, int past_len, int n_query, int num_q_heads,
+                           int num_kv_heads, int d, const float* centroids, int key_bits, int value_bits,
+                           float scale, int v_flags, int window, void* workspace, int64_t workspace_bytes,
+                           void* out, int out_dtype, const float* rotation, void* stream);
+
+/*
  * Store n_tokens x num_kv_heads K/V vectors ([n][Hkv][d], dtype) as fp16
  * (round to nearest even) into their raw slots; slot_mapping[i] < 0 skips
  * token i (and a slot past the cache is skipped too).  Replaces _store_raw_kv
