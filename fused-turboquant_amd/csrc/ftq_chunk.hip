@@ -270,7 +270,7 @@ hipError_t chunk_launch(const ChunkPlan& p, const void* q, int qt, int64_t q_row
   float* qfac = reinterpret_cast<float*>(ws + p.o_f);
   const int total = past + nq;
   const float qscale = (raw || rot != nullptr ? 1.f : fwht_scale(D)) * scale * 1.4426950408889634f;
-  hipError_t e = launch_chunk_query<D, 2, KHL>(q, qt, q_row, q_head, nq, hq, hkv, nullptr, rot, raw ? 0 : 1, qscale, qf,
+  hipError_t e = launch_chunk_query<D, 2, KHL>(q, qt, 0, q_row, q_head, nq, hq, hkv, hq, nullptr, rot, raw ? 0 : 1, qscale, qf,
                                                p.qstride, qfac, (int)p.colpad, st);
   if (e != hipSuccess) return e;
   a.kf = reinterpret_cast<const u32x4*>(kf);
@@ -285,7 +285,8 @@ hipError_t chunk_launch(const ChunkPlan& p, const void* q, int qt, int64_t q_row
   a.wl = direct ? nullptr : reinterpret_cast<float*>(ws + p.o_l);
   a.out = out; a.ot = ot; a.rot = vrot ? ROT_PLAIN : ROT_NONE; a.signs = nullptr;
   a.oscale = vrot ? fwht_scale(D) : 1.f;
-  a.o_row = o_row; a.o_head = o_head;
+  a.lens = nullptr; a.lens_less = 0; a.hkv_b = hkv;
+  a.o_batch = 0; a.o_row = o_row; a.o_head = o_head;
   const V1Geom geo = raw ? V1Geom{2 * D, 2 * D, 2 * D, 4 * D} : v1_geom(D, kb, vb, (flags & V1F_KFP8) != 0);
   const int wide = (((uintptr_t)cache | (uintptr_t)sblk | (uintptr_t)spos | (uintptr_t)shead) & 15) == 0;  // 16-byte slots
   const int pitch = ((geo.raw + 3) / 4 + 1) | 1;  // a pad dword, odd
@@ -299,7 +300,7 @@ hipError_t chunk_launch(const ChunkPlan& p, const void* q, int qt, int64_t q_row
         cache, nb, lbs, sblk, spos, shead, bt, mb, cent, kb, vb, (flags & V1F_KFP8) != 0, a.seg0, total, pitch, wide, kf,
         p.kstride, vf, p.vstride, tok, p.tstride);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    chunk_attn_kernel<D, 2, KHL, true><<<dim3((unsigned)(hkv * (p.colpad / p.cols)), p.splits), dim3(256), 0, st>>>(a);
+    chunk_attn_kernel<D, 2, KHL, false, true><<<dim3((unsigned)(hkv * (p.colpad / p.cols)), p.splits), dim3(256), 0, st>>>(a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (direct) return hipSuccess;

@@ -19,7 +19,7 @@
 // Fragment order: lane (m, g) of v_mfma_f32_16x16x32_f16 (m = lane & 15,
 // g = lane >> 4) reads 16 contiguous bytes, and a wave 1 KB:
 //   K  [16-token tile][32-dim step s][part][lane]: token m, dims 32 s + 8 g + j
-//   V  [32-token tile][16-dim block b][lane]: dim 16 b + m, tokens 4 g + j and
+//   V  [32-token tile][16-dim block b][part][lane]: dim 16 b + m, tokens 4 g + j and
 //      16 + 4 g + j (j < 4) -- the row order of the S^T accumulators, so P goes
 //      from the score registers into the P.V operand without a shuffle
 //   Q  [16-column tile][s][part][lane]: column m, dims 32 s + 8 g + j
@@ -49,7 +49,9 @@ struct ChunkAttn {
   int64_t kstride, vstride, qstride;  // uint4 per kv head
   int64_t tstride;             // floats per kv head
   int cstride;                 // columns per kv head (qfac)
-  int nq, G, hq, hkv, past, window;
+  int nq, G, hq, hkv, past, window;  // hq, hkv: of all sequences; past: the longest, for the grid
+  const int32_t* lens;         // per sequence, past = lens[b] - lens_less; null: one sequence, `past`
+  int hkv_b, lens_less;        // kv heads of one sequence
   int seg0, seg1;              // token range held by the fragments (seg0 a multiple of 64)
   int splits, split0, splits_all;  // splits of this launch, its first split, all splits of the row
   float *wo, *wl;              // partial outputs / log-sum-exps, or
@@ -57,7 +59,7 @@ struct ChunkAttn {
   int ot, rot;                 // output dtype; MergeRot of the direct output (ROT_NONE / PLAIN / SIGNS)
   const float* signs;
   float oscale;                // V fragments' common scale, and of the un-rotation (direct output only)
-  int64_t o_row, o_head;       // output strides (elements) of a query row and of a head
+  int64_t o_batch, o_row, o_head;  // output strides (elements) of a sequence, a query row and a head
 };
 
 // x of the lane 16 (32) lanes up or down: the butterfly pair of lane bit 4 (5)
@@ -84,15 +86,18 @@ __device__ __forceinline__ float f16_rest(float x, uint32_t w, int half) {
 
 // D: head dim; NH: f16 parts of the query and of the weights (2: ~22 bits, as
 // the v1 decode kernels; 1: f16); KHL: K fragments as hi + lo and the query
-// scaled per column (formats whose decode runs fp32 products); ZM: V has a
-// per-token minimum, and positions may lack a page.
-template <int D, int NH, bool KHL, bool ZM>
+// scaled per column (formats whose decode runs fp32 products); VHL: V
+// fragments as hi + lo (Lloyd-Max V at that precision); ZM: V has a per-token
+// minimum, and positions may be hidden by their bias.
+template <int D, int NH, bool KHL, bool VHL, bool ZM>
 __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
   using C = ChunkGeo<D, KHL>;
   constexpr int CT = C::CT, TK = C::TK, NS = C::NS, NB = C::NB, NT = C::NT, NP = C::NP;
   constexpr int KP = KHL ? 2 : 1;
-  constexpr int KU = NT * NS * KP * 64, VU = NP * NB * 64;  // 16-byte units of a tile
-  constexpr int KT = KU / 256 / KP, VT = VU / 256;
+  constexpr int VP = VHL ? 2 : 1;
+  static_assert(!VHL || KHL, "V hi + lo goes with K hi + lo");
+  constexpr int KU = NT * NS * KP * 64, VU = NP * NB * VP * 64;  // 16-byte units of a tile
+  constexpr int KT = KU / 256 / KP, VT = VU / 256 / VP;
   __shared__ u32x4 kb[2][KU];
   __shared__ u32x4 vb[2][VU];
   __shared__ __attribute__((aligned(16))) float tb[2][4][TK];
@@ -105,26 +110,28 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int n = lane & 15, g = lane >> 4;
   const int ncols = a.nq * a.G;
+  const int seq = kvh / a.hkv_b;
+  const int past = a.lens != nullptr ? a.lens[seq] - a.lens_less : a.past;
 
   // the rows of this workgroup, wave and lane
   const int c0 = blk * C::COLS;
   const int r_lo = c0 / a.G, r_hi = (min(c0 + C::COLS, ncols) - 1) / a.G;
   const int wc0 = c0 + wave * 16 * CT;
   const int wr_lo = min(wc0 / a.G, a.nq - 1), wr_hi = min((wc0 + 16 * CT - 1) / a.G, a.nq - 1);
-  const int first = a.window > 0 ? max(0, a.past + r_lo + 1 - a.window) : 0;
+  const int first = a.window > 0 ? max(0, past + r_lo + 1 - a.window) : 0;
   const int t0 = max(first, a.seg0) / TK;
-  const int t1 = (min(a.past + r_hi + 1, a.seg1) + TK - 1) / TK;
+  const int t1 = (min(past + r_hi + 1, a.seg1) + TK - 1) / TK;
   const int nt = t1 > t0 ? t1 - t0 : 0;
   const int per = (nt + a.splits - 1) / a.splits;
   const int tb0 = t0 + split * per, tb1 = min(tb0 + per, t1);
   // positions every / any row of the wave attends
-  const int w_all = a.past + wr_lo + 1;                                     // below: in every row's causal range
-  const int w_from = a.window > 0 ? max(0, a.past + wr_hi + 1 - a.window) : 0;  // from: in every row's window
+  const int w_all = past + wr_lo + 1;                                     // below: in every row's causal range
+  const int w_from = a.window > 0 ? max(0, past + wr_hi + 1 - a.window) : 0;  // from: in every row's window
   int lim[CT], lo[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int r = min((wc0 + 16 * ct + n) / a.G, a.nq - 1);
-    lim[ct] = a.past + r + 1;
+    lim[ct] = past + r + 1;
     lo[ct] = a.window > 0 ? max(0, lim[ct] - a.window) : 0;
   }
 
@@ -132,7 +139,7 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
   const u32x4* vf = a.vf + (int64_t)kvh * a.vstride;
   const float* tk = a.tok + (int64_t)kvh * a.tstride;
   const int tseg = a.seg0 / TK;
-  u32x4 rk[KT], rl[KHL ? KT : 1], rv[VT];
+  u32x4 rk[KT], rl[KHL ? KT : 1], rv[VT], rw[VHL ? VT : 1];
   float rt = 0.f;
   auto fetch = [&](int t) __attribute__((always_inline)) {
     const u32x4* pk = kf + (int64_t)(t - tseg) * KU + tid;
@@ -145,6 +152,10 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
     }
 #pragma unroll
     for (int j = 0; j < VT; ++j) rv[j] = pv[256 * j];
+    if constexpr (VHL) {
+#pragma unroll
+      for (int j = 0; j < VT; ++j) rw[j] = pv[256 * (VT + j)];
+    }
     if (tid < 4 * TK) rt = tk[(int64_t)(t - tseg) * 4 * TK + tid];
   };
   auto commit = [&](int p) __attribute__((always_inline)) {
@@ -156,6 +167,10 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
     }
 #pragma unroll
     for (int j = 0; j < VT; ++j) vb[p][tid + 256 * j] = rv[j];
+    if constexpr (VHL) {
+#pragma unroll
+      for (int j = 0; j < VT; ++j) vb[p][tid + 256 * (VT + j)] = rw[j];
+    }
     if (tid < 4 * TK) (&tb[p][0][0])[tid] = rt;
   };
 
@@ -174,7 +189,7 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
     qs[ct] = KHL ? a.qfac[(int64_t)kvh * a.cstride + wc0 + 16 * ct + n] : 1.f;
   }
 
-  constexpr float TAU = 8.f;        // weights stay below 2^TAU
+  constexpr float TAU = 4.f;        // weights stay below 2^TAU
   constexpr float MINF = -3.0e38f;  // running maximum of a column with no position yet
   float m_run[CT], l_run[CT], z_run[CT];
   floatx4 acc[CT][NB];
@@ -306,7 +321,13 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
     for (int k = 0; k < NP; ++k)
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        const half8 x = __builtin_bit_cast(half8, vb[p][(k * NB + b) * 64 + lane]);
+        const half8 x = __builtin_bit_cast(half8, vb[p][((k * NB + b) * VP) * 64 + lane]);
+        if constexpr (VHL) {
+          const half8 z = __builtin_bit_cast(half8, vb[p][((k * NB + b) * VP + 1) * 64 + lane]);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+            acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(z, __builtin_bit_cast(half8, ph[k][ct]), acc[ct][b], 0, 0, 0);
+        }
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
           acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8, ph[k][ct]), acc[ct][b], 0, 0, 0);
@@ -377,7 +398,7 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
           }
     }
     if (live) {
-      const int64_t off = (int64_t)r * a.o_row + (int64_t)h * a.o_head;
+      const int64_t off = seq * a.o_batch + (int64_t)r * a.o_row + (int64_t)(h - seq * a.hkv_b * a.G) * a.o_head;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         float o[4];
@@ -400,8 +421,8 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
 // [256, 512), so that the low parts of the others stay normal f16 numbers;
 // qfac takes the inverse.
 template <int D, int QT, int NH, bool KHL>
-__global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict__ query, int64_t q_row, int64_t q_head,
-                                                          int nq, int hq, int hkv, const float* __restrict__ signs,
+__global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict__ query, int64_t q_batch,
+                                                          int64_t q_row, int64_t q_head, int nq, int hq, int hkv, int hq_b, const float* __restrict__ signs,
                                                           const float* __restrict__ rot, int rotate, float qscale,
                                                           uint2* __restrict__ qf, int64_t qstride2,
                                                           float* __restrict__ qfac, int cstride) {
@@ -413,7 +434,8 @@ __global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict
   const int r = live ? (int)(v / hq) : 0, head = live ? (int)(v - (int64_t)r * hq) : 0;
   const int G = hq / hkv, kvh = head / G, col = r * G + head - kvh * G;
   float y[E];
-  load_elems<QT, E>(query, (int64_t)r * q_row + (int64_t)head * q_head + l16 * E, y);
+  const int seq = head / hq_b;
+  load_elems<QT, E>(query, seq * q_batch + (int64_t)r * q_row + (int64_t)(head - seq * hq_b) * q_head + l16 * E, y);
   if (signs != nullptr) {
 #pragma unroll
     for (int i = 0; i < E; ++i) y[i] *= signs[l16 * E + i];
@@ -456,14 +478,15 @@ __global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict
 }
 
 template <int D, int NH, bool KHL>
-hipError_t launch_chunk_query(const void* query, int qt, int64_t q_row, int64_t q_head, int nq, int hq, int hkv,
+hipError_t launch_chunk_query(const void* query, int qt, int64_t q_batch, int64_t q_row, int64_t q_head, int nq, int hq,
+                              int hkv, int hq_b,
                               const float* signs, const float* rot, int rotate, float qscale, uint4* qf,
                               int64_t qstride, float* qfac, int cstride, hipStream_t st) {
   const dim3 grid((unsigned)(((int64_t)nq * hq + 15) / 16)), block(256);
   uint2* q2 = reinterpret_cast<uint2*>(qf);
-  if (qt == F32) chunk_query_kernel<D, F32, NH, KHL><<<grid, block, 0, st>>>(query, q_row, q_head, nq, hq, hkv, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
-  else if (qt == F16) chunk_query_kernel<D, F16, NH, KHL><<<grid, block, 0, st>>>(query, q_row, q_head, nq, hq, hkv, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
-  else chunk_query_kernel<D, BF16, NH, KHL><<<grid, block, 0, st>>>(query, q_row, q_head, nq, hq, hkv, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
+  if (qt == F32) chunk_query_kernel<D, F32, NH, KHL><<<grid, block, 0, st>>>(query, q_batch, q_row, q_head, nq, hq, hkv, hq_b, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
+  else if (qt == F16) chunk_query_kernel<D, F16, NH, KHL><<<grid, block, 0, st>>>(query, q_batch, q_row, q_head, nq, hq, hkv, hq_b, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
+  else chunk_query_kernel<D, BF16, NH, KHL><<<grid, block, 0, st>>>(query, q_batch, q_row, q_head, nq, hq, hkv, hq_b, signs, rot, rotate, qscale, q2, 2 * qstride, qfac, cstride);
   return hipGetLastError();
 }
 

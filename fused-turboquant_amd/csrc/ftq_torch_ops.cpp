@@ -278,6 +278,99 @@ void v1_chunk_attention(const at::Tensor& query, const at::Tensor& kv_cache, con
       rotation.has_value() ? rotation->data_ptr<float>() : nullptr, stream_of(query)));
 }
 
+// ---- library-format attention: windows, other head dims, several tokens ----
+
+void lib_attention(const at::Tensor& query, const at::Tensor& codes_k, const std::optional<at::Tensor>& codes_v,
+                   const std::optional<at::Tensor>& norms_k, const std::optional<at::Tensor>& norms_v,
+                   const std::optional<at::Tensor>& block_table, const at::Tensor& lens,
+                   const std::optional<at::Tensor>& new_key, const std::optional<at::Tensor>& new_value,
+                   const at::Tensor& k_signs, const at::Tensor& v_signs, const at::Tensor& k_levels,
+                   const at::Tensor& v_levels, int64_t bits_k, int64_t bits_v, int64_t max_len, double scale,
+                   int64_t window, int64_t sinks, bool precise, at::Tensor& out) {
+  on_device(query, "query");
+  on_device(out, "out");
+  contig(codes_k, "codes_k");
+  contig(lens, "lens");
+  TORCH_CHECK(query.dim() == 4 && out.sizes() == query.sizes() && query.stride(3) == 1 && out.stride(3) == 1,
+              "fused_tq: query and out must be [B, Hq, n, d] with contiguous rows");
+  TORCH_CHECK(lens.scalar_type() == at::kInt && lens.numel() == query.size(0), "fused_tq: lens must be int32 [B]");
+  TORCH_CHECK(codes_k.scalar_type() == at::kByte && codes_k.dim() == 4, "fused_tq: codes_k must be uint8, 4-D");
+  TORCH_CHECK_VALUE(max_len >= 0 && max_len <= INT32_MAX && window >= 0 && window <= INT32_MAX && sinks >= 0 &&
+                        sinks <= INT32_MAX && query.size(2) <= INT32_MAX && query.size(0) <= INT32_MAX,
+                    "fused_tq: max_len / window / sinks out of range");
+  const bool paged = block_table.has_value();
+  const int64_t B = query.size(0), d = query.size(3), hkv = codes_k.size(1);
+  ftq_lib_attention_args a{};
+  a.query = query.data_ptr();
+  a.out = out.data_ptr();
+  a.q_batch = query.stride(0); a.q_head = query.stride(1); a.q_row = query.stride(2);
+  a.o_batch = out.stride(0); a.o_head = out.stride(1); a.o_row = out.stride(2);
+  a.q_dtype = dt(query); a.out_dtype = dt(out);
+  a.batch = (int)B; a.n_query = (int)query.size(2); a.num_q_heads = (int)query.size(1); a.num_kv_heads = (int)hkv;
+  a.d = (int)d;
+  a.paged = paged ? 1 : 0;
+  a.codes_k = codes_k.data_ptr<uint8_t>();
+  if (paged) {
+    contig(*block_table, "block_table");
+    TORCH_CHECK(block_table->scalar_type() == at::kInt && block_table->dim() == 2 && block_table->size(0) == B,
+                "fused_tq: block_table must be int32 [B, max_blocks]");
+    TORCH_CHECK(codes_k.size(3) == 2 * d * (bits_k + bits_v) + 64, "fused_tq: sub-block size does not match (d, bits)");
+    a.block_table = block_table->data_ptr<int32_t>();
+    a.page_size = (int)codes_k.size(2) * 16; a.max_blocks = (int)block_table->size(1); a.num_blocks = codes_k.size(0);
+  } else {
+    TORCH_CHECK(codes_v.has_value() && norms_k.has_value() && norms_v.has_value(), "fused_tq: flat codes and norms");
+    contig(*codes_v, "codes_v");
+    contig(*norms_k, "norms_k");
+    contig(*norms_v, "norms_v");
+    const int64_t cap = codes_k.size(2);
+    TORCH_CHECK(codes_k.size(0) == B && codes_k.size(3) == d * bits_k / 8 && codes_v->scalar_type() == at::kByte &&
+                    codes_v->dim() == 4 && codes_v->size(0) == B && codes_v->size(1) == hkv && codes_v->size(2) == cap &&
+                    codes_v->size(3) == d * bits_v / 8,
+                "fused_tq: flat codes must be [B, Hkv, capacity, d * bits / 8]");
+    TORCH_CHECK(norms_k->scalar_type() == at::kHalf && norms_v->scalar_type() == at::kHalf &&
+                    norms_k->numel() == B * hkv * cap && norms_v->numel() == B * hkv * cap,
+                "fused_tq: flat norms must be float16 [B, Hkv, capacity]");
+    a.codes_v = codes_v->data_ptr<uint8_t>();
+    a.norms_k = reinterpret_cast<const uint16_t*>(norms_k->data_ptr());
+    a.norms_v = reinterpret_cast<const uint16_t*>(norms_v->data_ptr());
+    a.capacity = (int)cap;
+  }
+  a.lens = lens.data_ptr<int32_t>();
+  a.max_len = (int)max_len;
+  for (const at::Tensor* t : {&k_signs, &v_signs}) {
+    contig(*t, "signs");
+    TORCH_CHECK(t->numel() == d, "fused_tq: signs must have d entries");
+  }
+  contig(k_levels, "k_levels");
+  contig(v_levels, "v_levels");
+  TORCH_CHECK(bits_k >= 2 && bits_k <= 4 && bits_v >= 2 && bits_v <= 4 && k_levels.numel() == (1 << bits_k) &&
+                  v_levels.numel() == (1 << bits_v),
+              "fused_tq: levels must have 2^bits entries");
+  a.k_signs = k_signs.data_ptr<float>(); a.v_signs = v_signs.data_ptr<float>();
+  a.k_levels = k_levels.data_ptr<float>(); a.v_levels = v_levels.data_ptr<float>();
+  a.bits_k = (int)bits_k; a.bits_v = (int)bits_v;
+  if (new_key.has_value()) {
+    TORCH_CHECK(new_value.has_value() && new_key->dim() == 4 && new_key->sizes() == new_value->sizes() &&
+                    new_key->size(0) == B && new_key->size(1) == hkv && new_key->size(2) == query.size(2) &&
+                    new_key->size(3) == d && new_key->stride(3) == 1 && new_value->stride(3) == 1 &&
+                    new_key->scalar_type() == new_value->scalar_type(),
+                "fused_tq: new keys and values must be [B, Hkv, n, d] with contiguous rows");
+    on_device(*new_key, "new_key");
+    on_device(*new_value, "new_value");
+    a.new_key = new_key->data_ptr(); a.new_value = new_value->data_ptr(); a.new_dtype = dt(*new_key);
+    a.k_batch = new_key->stride(0); a.k_head = new_key->stride(1); a.k_tok = new_key->stride(2);
+    a.v_batch = new_value->stride(0); a.v_head = new_value->stride(1); a.v_tok = new_value->stride(2);
+  }
+  a.scale = (float)scale; a.window = (int)window; a.sinks = (int)sinks; a.precise = precise ? 1 : 0;
+  const c10::DeviceGuard g(query.device());
+  if (B == 0 || query.size(2) == 0) return;
+  const int64_t need = ftq_lib_attention_workspace_bytes(a.batch, a.n_query, a.num_q_heads, a.num_kv_heads, a.d,
+                                                         a.max_len, a.window, a.sinks, a.precise, a.new_key == nullptr);
+  TORCH_CHECK_VALUE(need >= 0, "fused_tq: library attention does not take these sizes");
+  at::Tensor ws = at::empty({need}, query.options().dtype(at::kByte));
+  check_rc(ftq_lib_attention(&a, ws.data_ptr(), need, stream_of(query)));
+}
+
 // ---- raw fp16 slots (boundary layers) -------------------------------------
 
 void raw_store(const at::Tensor& key, const at::Tensor& value, at::Tensor& kv_cache, const at::Tensor& slot_mapping) {
@@ -340,6 +433,10 @@ TORCH_LIBRARY(fused_tq, m) {
         "int num_splits, Tensor(a!) workspace, Tensor(b!) out, Tensor(c!)? lse, Tensor? rotation) -> ()");
   m.def("v1_chunk_attention(Tensor query, Tensor kv_cache, Tensor block_row, int past_len, Tensor? centroids, "
         "int key_bits, int value_bits, float scale, int v_flags, int window, Tensor(a!) out, Tensor? rotation) -> ()");
+  m.def("lib_attention(Tensor query, Tensor codes_k, Tensor? codes_v, Tensor? norms_k, Tensor? norms_v, "
+        "Tensor? block_table, Tensor lens, Tensor? new_key, Tensor? new_value, Tensor k_signs, Tensor v_signs, "
+        "Tensor k_levels, Tensor v_levels, int bits_k, int bits_v, int max_len, float scale, int window, int sinks, "
+        "bool precise, Tensor(a!) out) -> ()");
   m.def("raw_store(Tensor key, Tensor value, Tensor(a!) kv_cache, Tensor slot_mapping) -> ()");
   m.def("raw_decode_attention(Tensor query, Tensor kv_cache, Tensor block_table, Tensor seq_lens, "
         "Tensor? kv_start, float scale, int num_splits, Tensor(a!) workspace, Tensor(b!) out, "
@@ -356,6 +453,7 @@ TORCH_LIBRARY_IMPL(fused_tq, CUDA, m) {
   m.impl("v1_store", &v1_store);
   m.impl("v1_decode_attention", &v1_decode_attention);
   m.impl("v1_chunk_attention", &v1_chunk_attention);
+  m.impl("lib_attention", &lib_attention);
   m.impl("raw_store", &raw_store);
   m.impl("raw_decode_attention", &raw_decode_attention);
 }

@@ -51,7 +51,7 @@ def _register_fakes() -> None:
 
     # operators that only write their (a!) arguments
     for name in ("paged_store", "paged_decode_attention", "v1_store", "v1_decode_attention",
-                 "v1_chunk_attention", "raw_store", "raw_decode_attention"):
+                 "v1_chunk_attention", "lib_attention", "raw_store", "raw_decode_attention"):
         torch.library.register_fake(lib + name)(lambda *args, **kwargs: None)
 
 

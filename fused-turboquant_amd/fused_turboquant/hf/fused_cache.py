@@ -299,14 +299,18 @@ class CompressedKVCache(DynamicCache):
     def decode_attention(self, query: torch.Tensor, layer_idx: int, scale: float,
                          sliding_window: Optional[int] = None, sink_tokens: int = 0) -> torch.Tensor:
         """query [B, Hq, d] -> [B, Hq, d] (query dtype): the fused paged decode
-        attention; for flat (non-paged) layers and sliding windows, softmax
-        attention in fp32 over the decoded K / V of each sequence's positions
-        (with a window: the last ``sliding_window`` and the first
-        ``sink_tokens``, reference ``hf/fused_cache.py:600-611``)."""
+        attention; for flat (non-paged) layers and sliding windows the
+        library-format attention kernels, at float32-level products (with a
+        window: the last ``sliding_window`` positions and the first
+        ``sink_tokens``, reference ``hf/fused_cache.py:600-611``), or, at head
+        dims without one, softmax attention in fp32 over the decoded K / V."""
         lp = self._pages[layer_idx]
         if isinstance(lp, _LayerPages) and sliding_window is None:
             return P.paged_decode_attention(query, lp.kv_cache, lp.block_table, lp.lens_dev, lp.k_tq, lp.v_tq,
                                             scale=scale, max_seq_len=max(lp.lens))
+        if self._fused_attention(lp, query):
+            return self._lib_attention(lp, query.unsqueeze(2), scale, window=sliding_window,
+                                       sinks=sink_tokens).squeeze(2)
         kd = self.decode_keys(layer_idx)
         vd = self.decode_values(layer_idx)
         B, hq, d = query.shape
@@ -323,6 +327,32 @@ class CompressedKVCache(DynamicCache):
         w = torch.softmax(scores, dim=-1)
         w = torch.nan_to_num(w, nan=0.0)  # a sequence with no positions gives 0
         return torch.matmul(w, _repeat_kv(vd, n_rep)).squeeze(2).to(query.dtype)
+
+    @staticmethod
+    def _fused_attention(lp, query: torch.Tensor) -> bool:
+        """Whether the library-format attention kernels take this layer and query."""
+        hq, d = query.shape[1], query.shape[-1]
+        return (d == lp.d and d in P.LIB_ATTENTION_DIMS and hq % lp.hkv == 0 and hq // lp.hkv <= 16
+                and lp.B * lp.hkv <= 65535 and query.dtype in (torch.float32, torch.float16, torch.bfloat16))
+
+    @staticmethod
+    def _lib_attention(lp, query: torch.Tensor, scale: float, new_kv=None, window=None, sinks: int = 0):
+        src = (dict(pages=(lp.kv_cache, lp.block_table)) if isinstance(lp, _LayerPages)
+               else dict(flat=(lp.kp, lp.kn, lp.vp, lp.vn)))
+        return P.lib_attention(query, lp.lens_dev, max(lp.lens), lp.k_tq, lp.v_tq, scale, new_kv=new_kv,
+                               window=window, sinks=sinks, **src)
+
+    def chunk_attention(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, layer_idx: int,
+                        scale: float, sliding_window: Optional[int] = None) -> Optional[torch.Tensor]:
+        """Attention of a multi-token step whose keys / values [B, Hkv, q, d]
+        have just been stored for every token: query [B, Hq, q, d] over the
+        compressed past and the step's own tokens, causal.  None where the
+        kernels do not take the layer."""
+        lp = self._pages[layer_idx]
+        if not self._fused_attention(lp, query) or key.dtype != value.dtype or key.dtype not in (
+                torch.float32, torch.float16, torch.bfloat16):
+            return None
+        return self._lib_attention(lp, query, scale, new_kv=(key, value), window=sliding_window)
 
     def reset(self):
         """Drop every layer so the object can serve a new prompt (reference :350-360)."""
@@ -531,6 +561,9 @@ def make_fused_attention_forward(attn_module, cache: CompressedKVCache, quantize
                 mask = (i[None, :] <= i[:, None]) & (i[None, :] > i[:, None] - window)
             out = F.scaled_dot_product_attention(q, _repeat_kv(k, n_rep), _repeat_kv(v, n_rep),
                                                  attn_mask=mask, scale=scale, is_causal=mask is None)
+        elif compress_v and keep is None and (
+                fused := cache.chunk_attention(q, k, v, layer_idx, scale, sliding_window=window)) is not None:
+            out = fused  # the compressed past and the new tokens, one pass of the kernels
         else:
             # new tokens attend over the decoded past and themselves (causal)
             kd = cache.decode_keys(layer_idx)[:, :, :past_len].to(q.dtype)

@@ -178,6 +178,55 @@ def paged_decode_attention(query: torch.Tensor, kv_cache: torch.Tensor, block_ta
     return out
 
 
+LIB_ATTENTION_DIMS = (64, 128, 256)  # head dims of ``lib_attention``
+
+
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    """``t`` with rows the kernels can read in 16-byte steps (itself where it has them)."""
+    if t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0:
+        return t
+    return t.contiguous()
+
+
+def lib_attention(query: torch.Tensor, lens: torch.Tensor, max_len: int, k_quant: TurboQuantMSE,
+                  v_quant: TurboQuantMSE, scale: float, pages: tuple | None = None, flat: tuple | None = None,
+                  new_kv: tuple | None = None, window: int | None = None, sinks: int = 0,
+                  precise: bool | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+    """Attention of query [B, Hq, n, d] (d = 64, 128 or 256) over a
+    library-format cache, ``pages = (kv_cache, block_table)`` or ``flat =
+    (k_codes, k_norms, v_codes, v_norms)`` (``CompressedTensor`` rows, [B, Hkv,
+    capacity, ...]); ``lens`` int32 [B] positions, ``max_len`` their maximum.
+
+    Without ``new_kv``: one query token per sequence over the last ``window``
+    positions and the first ``sinks`` (no window: over all).  With ``new_kv =
+    (key, value)`` [B, Hkv, n, d], the step's own tokens (already counted in
+    ``lens``): row i attends the compressed past, the new tokens up to its own
+    as given, and of these with a window only its last ``window``.
+    ``precise`` (default: without ``new_kv``, or for float32 queries) keeps
+    float32-level products; otherwise the operands are f16."""
+    if (pages is None) == (flat is None):
+        raise ValueError("pass pages or flat")
+    B, hq, n, d = query.shape
+    if lens.dtype != torch.int32 or lens.numel() != B:
+        raise ValueError("lens must be int32 [B]")
+    if precise is None:
+        precise = new_kv is None or query.dtype == torch.float32
+    q = _rows16(query)
+    if out is None:
+        out = torch.empty(B, n, hq, d, dtype=q.dtype, device=q.device).transpose(1, 2)
+    nk = nv = None
+    if new_kv is not None:
+        nk, nv = _rows16(new_kv[0]), _rows16(new_kv[1])
+    kq, vq = k_quant.quantizer, v_quant.quantizer
+    codes_k, codes_v, norms_k, norms_v, bt = ((pages[0], None, None, None, pages[1]) if pages is not None else
+                                              (flat[0], flat[2], flat[1], flat[3], None))
+    _lib.require_device(q, codes_k, lens, out)
+    _ops.ops().lib_attention(q, codes_k, codes_v, norms_k, norms_v, bt, lens, nk, nv, k_quant.rotation.signs,
+                             v_quant.rotation.signs, kq.levels, vq.levels, k_quant.bits, v_quant.bits, int(max_len),
+                             float(scale), int(window or 0), int(sinks) if window else 0, bool(precise), out)
+    return out
+
+
 _V_GATHER: dict = {}
 
 

@@ -409,6 +409,49 @@ int ftq_v1_chunk_attention(const void* query, int q_dtype, const uint8_t* kv_cac
                            void* out, int out_dtype, const float* rotation, void* stream);
 
 /*
+ * Attention over a library-format cache (pages of ftq_paged_store, or flat
+ * codes and norms per sequence) for the calls that
+ * ftq_paged_decode_attention does not take; d = 64, 128 or 256:
+ *   - a decode step (new_key null, n_query 1) over the last `window` positions
+ *     and the first `sinks` (window 0: every position);
+ *   - a multi-token step (new_key / new_value, n_query tokens per sequence,
+ *     already counted in lens): row i attends the compressed past, the new
+ *     tokens up to its own as they are, and with window > 0 only the last
+ *     `window` of these.
+ * Replaces the decode-the-cache-and-attend path of reference
+ * hf/fused_cache.py:576-670.  precise: f16 hi + lo operands (float32-level
+ * products); else f16 operands with fp32 sums.
+ */
+typedef struct {
+  const void* query;  /* [batch, num_q_heads, n_query, d], rows of d contiguous */
+  void* out;          /* the same shape */
+  int64_t q_batch, q_head, q_row, o_batch, o_head, o_row; /* strides in elements, multiples of 8 */
+  int q_dtype, out_dtype;
+  int batch, n_query, num_q_heads, num_kv_heads, d;
+  int paged;                /* 1: codes_k is the page pool; 0: flat rows */
+  const uint8_t* codes_k;   /* pages [num_blocks][Hkv][page_size / 16][sub-block], or [batch][Hkv][capacity][d bits_k / 8] */
+  const uint8_t* codes_v;   /* flat: [batch][Hkv][capacity][d bits_v / 8] */
+  const uint16_t* norms_k;  /* flat: fp16 [batch][Hkv][capacity] */
+  const uint16_t* norms_v;
+  const int32_t* block_table; /* pages: [batch][max_blocks]; every position below lens has a page */
+  int page_size, max_blocks, capacity;
+  int64_t num_blocks;
+  const int32_t* lens;      /* positions per sequence, the new tokens among them */
+  int max_len;              /* their maximum */
+  const float *k_signs, *v_signs, *k_levels, *v_levels;
+  int bits_k, bits_v;
+  const void* new_key;      /* [batch, num_kv_heads, n_query, d], or null */
+  const void* new_value;
+  int new_dtype;
+  int64_t k_batch, k_head, k_tok, v_batch, v_head, v_tok; /* strides in elements, multiples of 8 */
+  float scale;
+  int window, sinks, precise;
+} ftq_lib_attention_args;
+int64_t ftq_lib_attention_workspace_bytes(int batch, int n_query, int num_q_heads, int num_kv_heads, int d,
+                                          int max_len, int window, int sinks, int precise, int decode);
+int ftq_lib_attention(const ftq_lib_attention_args* args, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Store n_tokens x num_kv_heads K/V vectors ([n][Hkv][d], dtype) as fp16
  * (round to nearest even) into their raw slots; slot_mapping[i] < 0 skips
  * token i (and a slot past the cache is skipped too).  Replaces _store_raw_kv

@@ -1,0 +1,122 @@
+"""Library-format attention kernels (``paged.lib_attention`` through the
+HuggingFace cache): windowed and flat decode steps and multi-token steps,
+against float64 attention over the oracle's decode of the stored codes (and,
+for a multi-token step, the new tokens as given).
+
+Tolerances (relative 2-norm on fp32 outputs): decode steps and float32
+multi-token steps carry f16 hi + lo operands (2^-22) with fp32 sums: 1e-5.
+16-bit multi-token steps carry f16 operands, each with a relative error of at
+most 2^-11 (1e-3 on the outputs, whose own rounding is 2^-9 for bf16).
+"""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import tq_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _cache(cuda, d, bk, bv, B, hkv, lens, seed, dtype=torch.bfloat16):
+    from fused_turboquant import TurboQuantMSE
+    from fused_turboquant.hf import CompressedKVCache
+    g = torch.Generator().manual_seed(seed)
+    k_tq, v_tq = TurboQuantMSE(d, bits=bk, device=cuda), TurboQuantMSE(d, bits=bv, device=cuda)
+    cache = CompressedKVCache(k_tq)
+    cache.set_layer_quantizer(0, k_tq)
+    cache.set_layer_quantizer_v(0, v_tq)
+    L = max(lens)
+    k, v = (torch.randn(B, hkv, L, d, generator=g) for _ in range(2))
+    k[:, :, ::29] *= 5.0
+    keep = torch.tensor([[i >= L - n for i in range(L)] for n in lens], device=cuda)
+    cache.store_compressed_kv(k.to(dtype).to(cuda), v.to(dtype).to(cuda), 0, keep=None if all(n == L for n in lens) else keep)
+    return cache, g
+
+
+def _decoded(cache, which, B, hkv, d):
+    e = cache.get_compressed_key(0) if which == "k" else cache.get_compressed_value(0)
+    tq = cache.get_layer_quantizer(0) if which == "k" else cache.get_layer_quantizer_v(0)
+    S = e["packed_indices"].shape[2]
+    x = O.decode(e["packed_indices"].cpu().numpy().reshape(-1, d * tq.bits // 8), e["norms"].cpu().numpy().reshape(-1),
+                 tq.quantizer.levels.cpu().numpy(), tq.rotation.signs.cpu().numpy(), tq.bits, d)
+    return x.reshape(B, hkv, S, d).astype(np.float64)
+
+
+def _attend(q, k, v, scale, ok):
+    """q [n, d], k / v [S, d], ok [n, S] -> [n, d], float64."""
+    s = np.where(ok, q @ k.T * scale, -np.inf)
+    p = np.exp(s - s.max(axis=1, keepdims=True))
+    return (p / p.sum(axis=1, keepdims=True)) @ v
+
+
+def _rel(got, want):
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("d,bk,bv,B,hkv,G,lens,window,sinks", [
+    (128, 4, 4, 2, 2, 4, (300, 300), 100, 4),    # the window starts inside a page
+    (128, 3, 2, 1, 2, 7, (97,), 33, 40),         # more sinks than one tile
+    (256, 4, 3, 2, 1, 2, (200, 150), 64, 4),     # sequences of different lengths
+    (128, 2, 4, 2, 2, 1, (40, 17), 512, 4),      # a window longer than the context
+    (64, 4, 4, 2, 2, 4, (130, 130), None, 0),    # flat rows, the whole context
+    (64, 3, 3, 3, 2, 16, (70, 33, 1), 32, 4),    # flat rows, a window, short sequences
+    (64, 2, 4, 1, 1, 8, (2100,), 1000, 4),       # splits over the context
+])
+def test_decode_step(cuda, d, bk, bv, B, hkv, G, lens, window, sinks):
+    cache, g = _cache(cuda, d, bk, bv, B, hkv, lens, seed=d + bk)
+    q = torch.randn(B, hkv * G, d, generator=g)
+    got = cache.decode_attention(q.to(cuda), 0, 1 / math.sqrt(d), sliding_window=window, sink_tokens=sinks).cpu().numpy()
+    kd, vd = _decoded(cache, "k", B, hkv, d), _decoded(cache, "v", B, hkv, d)
+    want = np.zeros(got.shape)
+    for b, n in enumerate(lens):
+        pos = np.arange(n)
+        ok = np.ones(n, bool) if window is None else (pos >= n - window) | (pos < sinks)
+        for h in range(hkv * G):
+            want[b, h] = _attend(q[b, h:h + 1].double().numpy(), kd[b, h // G, :n], vd[b, h // G, :n], 1 / math.sqrt(d), ok[None])[0]
+    err = _rel(got, want)
+    print(f"[lib decode d{d} K{bk}V{bv} lens {lens} w{window}] rel {err:.2e}", flush=True)
+    assert err < 1e-5
+
+
+@pytest.mark.parametrize("d,bk,bv,B,hkv,G,past,n,window,dtype", [
+    (128, 4, 4, 1, 2, 4, 200, 70, None, torch.bfloat16),   # past ends inside a tile
+    (128, 3, 2, 2, 2, 7, 64, 33, 50, torch.float16),       # a window over past and new tokens
+    (256, 4, 4, 2, 1, 2, 45, 20, None, torch.bfloat16),
+    (64, 4, 3, 2, 2, 4, 100, 65, None, torch.bfloat16),
+    (64, 4, 4, 1, 1, 16, 31, 2, 40, torch.float16),
+    (128, 4, 4, 1, 2, 4, 90, 40, None, torch.float32),
+    (64, 3, 3, 2, 1, 4, 33, 17, 20, torch.float32),
+    (256, 2, 4, 1, 2, 2, 64, 31, None, torch.float32),
+])
+def test_multi_token_step(cuda, d, bk, bv, B, hkv, G, past, n, window, dtype):
+    cache, g = _cache(cuda, d, bk, bv, B, hkv, (past,) * B, seed=d + past, dtype=dtype)
+    kd, vd = (np.ascontiguousarray(_decoded(cache, w, B, hkv, d)[:, :, :past]) for w in "kv")
+    k, v = (torch.randn(B, hkv, n, d, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(B, hkv * G, n, d, generator=g).to(dtype)
+    cache.store_compressed_kv(k.to(cuda), v.to(cuda), 0)
+    got = cache.chunk_attention(q.to(cuda), k.to(cuda), v.to(cuda), 0, 1 / math.sqrt(d), sliding_window=window)
+    assert got is not None and got.dtype == dtype and got.shape == q.shape
+    want = np.zeros(q.shape)
+    row, col = past + np.arange(n)[:, None], np.arange(past + n)[None]
+    ok = (col <= row) & (col > row - window) if window else col <= row
+    for b in range(B):
+        for h in range(hkv * G):
+            kk = np.concatenate([kd[b, h // G], k[b, h // G].double().numpy()])
+            vv = np.concatenate([vd[b, h // G], v[b, h // G].double().numpy()])
+            want[b, h] = _attend(q[b, h].double().numpy(), kk, vv, 1 / math.sqrt(d), ok)
+    err = _rel(got.float().cpu().numpy(), want)
+    print(f"[lib chunk d{d} K{bk}V{bv} past {past} n {n} w{window} {dtype}] rel {err:.2e}", flush=True)
+    assert err < {torch.float32: 1e-5, torch.float16: 1e-3 + 2.0 ** -11, torch.bfloat16: 1e-3 + 2.0 ** -9}[dtype]
+
+
+def test_large_values_stay_finite(cuda):
+    """New values up to what an fp16 norm holds, and zero vectors."""
+    cache, g = _cache(cuda, 64, 4, 4, 1, 1, (20,), seed=1)
+    k, v = torch.zeros(1, 1, 8, 64), torch.randn(1, 1, 8, 64, generator=g) * 5000.0
+    q = torch.randn(1, 4, 8, 64, generator=g)
+    dt = torch.bfloat16
+    cache.store_compressed_kv(k.to(dt).to(cuda), v.to(dt).to(cuda), 0)
+    got = cache.chunk_attention(q.to(dt).to(cuda), k.to(dt).to(cuda), v.to(dt).to(cuda), 0, 0.125)
+    assert torch.isfinite(got).all() and got.abs().max() > 1000
