@@ -22,10 +22,9 @@ constexpr int KB_RAW = 16;  // key_bits of raw fp16 slots
 
 // n <= 16 bits at bit offset p of a little-endian dword row (one pad dword)
 __device__ __forceinline__ uint32_t row_bits(const uint32_t* row, int p, int n) {
-  const int i = p >> 5, o = p & 31;
-  uint32_t v = row[i] >> o;
-  if (o + n > 32) v |= row[i + 1] << (32 - o);
-  return v & ((1u << n) - 1u);
+  // both words always (no branch, so that the reads of several codes overlap)
+  const int i = p >> 5;
+  return __builtin_amdgcn_alignbit(row[i + 1], row[i], (uint32_t)p & 31u) & ((1u << n) - 1u);
 }
 
 __device__ __forceinline__ float e4m3_value(uint32_t b) {

@@ -214,24 +214,60 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) sl[k][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
+    // All K fragments of the tile are requested at once (with hi + lo parts,
+    // the registers hold one step's), and V's right after the score products,
+    // so that one LDS latency is exposed per tile and V's lands during the
+    // softmax.  Independent accumulators alternate between dependent products.
+    half8 xk[KHL ? 1 : NS][NT];
+    if constexpr (!KHL) {
 #pragma unroll
-    for (int d = 0; d < NS; ++d)
+      for (int d = 0; d < NS; ++d)
 #pragma unroll
-      for (int k = 0; k < NT; ++k) {
-        half8 x = __builtin_bit_cast(half8, kb[p][((k * NS + d) * KP) * 64 + lane]);
+        for (int k = 0; k < NT; ++k) xk[d][k] = __builtin_bit_cast(half8, kb[p][(k * NS + d) * 64 + lane]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, qh[ct][d], s[k][ct], 0, 0, 0);
-          if constexpr (KHL) sl[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, ql[ct][d], sl[k][ct], 0, 0, 0);
-          else if constexpr (NH == 2) s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, ql[ct][d], s[k][ct], 0, 0, 0);
+    for (int d = 0; d < NS; ++d) {
+      if constexpr (KHL) {
+        half8 xh[NT], xl[NT];
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+          xh[k] = __builtin_bit_cast(half8, kb[p][((k * NS + d) * KP) * 64 + lane]);
+          xl[k] = __builtin_bit_cast(half8, kb[p][((k * NS + d) * KP + 1) * 64 + lane]);
         }
-        if constexpr (KHL) {
-          x = __builtin_bit_cast(half8, kb[p][((k * NS + d) * KP + 1) * 64 + lane]);
-  #pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-            sl[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, qh[ct][d], sl[k][ct], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[k], qh[ct][d], s[k][ct], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) sl[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[k], ql[ct][d], sl[k][ct], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) sl[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[k], qh[ct][d], sl[k][ct], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xk[d][k], qh[ct][d], s[k][ct], 0, 0, 0);
+        if constexpr (NH == 2) {
+#pragma unroll
+          for (int k = 0; k < NT; ++k)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) s[k][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xk[d][k], ql[ct][d], s[k][ct], 0, 0, 0);
         }
       }
+    }
+    constexpr bool VEARLY = !VHL && NP * NB <= 8;
+    half8 xv[VEARLY ? NP * NB : 1];
+    if constexpr (VEARLY) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NP * NB; ++i) xv[i] = __builtin_bit_cast(half8, vb[p][i * 64 + lane]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const bool edge = t * TK + TK > w_all || t * TK < w_from;  // wave-uniform
     // scores: x K factor (and the column's), + bias; masked on the edges
 #pragma unroll
@@ -320,20 +356,27 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
 #pragma unroll
     for (int k = 0; k < NP; ++k)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const half8 x = __builtin_bit_cast(half8, vb[p][((k * NB + b) * VP) * 64 + lane]);
-        if constexpr (VHL) {
-          const half8 z = __builtin_bit_cast(half8, vb[p][((k * NB + b) * VP + 1) * 64 + lane]);
+      for (int b0 = 0; b0 < NB; b0 += 2) {
+        half8 x[2], z[2];
 #pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-            acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(z, __builtin_bit_cast(half8, ph[k][ct]), acc[ct][b], 0, 0, 0);
+        for (int b = 0; b < 2; ++b) {
+          if constexpr (VEARLY) x[b] = xv[k * NB + b0 + b];
+          else x[b] = __builtin_bit_cast(half8, vb[p][((k * NB + b0 + b) * VP) * 64 + lane]);
+          if constexpr (VHL) z[b] = __builtin_bit_cast(half8, vb[p][((k * NB + b0 + b) * VP + 1) * 64 + lane]);
         }
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8, ph[k][ct]), acc[ct][b], 0, 0, 0);
-          if constexpr (NH == 2)
-            acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8, pl[k][ct]), acc[ct][b], 0, 0, 0);
-        }
+        for (int part = VHL ? -1 : 0; part < NH; ++part)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+              const half8 w = part < 0 ? z[b] : x[b];
+              u32x4 pw = ph[k][ct];
+              if constexpr (NH == 2) {
+                if (part == 1) pw = pl[k][ct];
+              }
+              acc[ct][b0 + b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, __builtin_bit_cast(half8, pw), acc[ct][b0 + b], 0, 0, 0);
+            }
       }
   };
 

@@ -45,12 +45,11 @@ struct LibSource {
   int window, sinks, vsinks;  // decode: window (0: none), sinks, and their virtual positions (a multiple of 32)
 };
 
-// bits [p, p + n) of a dword array, n <= 16
+// bits [p, p + n) of a dword array with a pad dword, n <= 16
 __device__ __forceinline__ uint32_t word_bits(const uint32_t* w, int p, int n) {
-  const int i = p >> 5, o = p & 31;
-  uint32_t v = w[i] >> o;
-  if (o + n > 32) v |= w[i + 1] << (32 - o);
-  return v & ((1u << n) - 1u);
+  // both words always (no branch, so that the reads of several codes overlap)
+  const int i = p >> 5;
+  return __builtin_amdgcn_alignbit(w[i + 1], w[i], (uint32_t)p & 31u) & ((1u << n) - 1u);
 }
 
 // One 32-token tile of one (sequence, kv head).  Virtual position v stands
