@@ -1469,7 +1469,8 @@ extern "C" int ftq_v1_choose_splits(int batch, int num_q_heads, int num_kv_heads
   if (batch <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0) return 1;
   const bool mfma = d == 128 && (v_flags & (V1F_KFP8 | V1F_FP32)) == 0 && key_bits >= 2 && key_bits <= 4 &&
                     value_bits >= 2 && value_bits <= 4;
-  if (!mfma) return ftq_v1_default_splits(batch, num_kv_heads, max_seq_len);
+  const bool split_ops = v1_split_takes(d, key_bits, value_bits, v_flags);
+  if (!mfma && !split_ops) return ftq_v1_default_splits(batch, num_kv_heads, max_seq_len);
   // The most splits whose grid the GPU holds in one round: past that a second
   // round of workgroups (or an uneven first one) costs more than the longer
   // tiles per wave.  Measured on 32 query / 8 kv heads, K3 V3 (3 workgroups
@@ -1481,7 +1482,8 @@ extern "C" int ftq_v1_choose_splits(int batch, int num_q_heads, int num_kv_heads
   const int group = num_q_heads / num_kv_heads;
   const bool lloyd = value_bits == 4 && (v_flags & V1F_VLM) != 0;
   int cap;
-  if (key_bits == 2) cap = v1_attn_resident_k<2>(value_bits, group, lloyd);
+  if (split_ops) cap = v1_split_resident(d);
+  else if (key_bits == 2) cap = v1_attn_resident_k<2>(value_bits, group, lloyd);
   else if (key_bits == 3) cap = v1_attn_resident_k<3>(value_bits, group, lloyd);
   else cap = v1_attn_resident_k<4>(value_bits, group, lloyd);
   const int64_t units = std::min<int64_t>((int64_t)batch * num_kv_heads, 1 << 20);
@@ -1558,11 +1560,13 @@ int v1_attn_launch(const V1Args& a, int d, int key_bits, int value_bits, int v_r
   hipStream_t st = (hipStream_t)stream;
   const bool kf8 = (v_rotate & V1F_KFP8) != 0;
   hipError_t e;
-  // the matrix-core kernels: head_dim 128, 2-4 bit codes, f16 operands; every
+  // the matrix-core kernels: head_dim 128, 2-4 bit codes, f16 operands; head_dim
+  // 64 / 256, 2-4 bit codes, operands split to float32-level products.  Every
   // other format, and fp32 products on request, on the VALU kernel
   const bool mfma = d == 128 && !kf8 && (v_rotate & V1F_FP32) == 0 && key_bits >= 2 && key_bits <= 4 &&
                     value_bits >= 2 && value_bits <= 4;
-  if (!mfma) e = v1_valu_launch(a, d, key_bits, value_bits, v_rotate, st);
+  if (v1_split_takes(d, key_bits, value_bits, v_rotate)) e = v1_split_launch(a, d, key_bits, value_bits, st);
+  else if (!mfma) e = v1_valu_launch(a, d, key_bits, value_bits, v_rotate, st);
   else if (key_bits == 2) e = v1_launch_attn2<128, 2>(value_bits, a, st);
   else if (key_bits == 3) e = v1_launch_attn2<128, 3>(value_bits, a, st);
   else e = v1_launch_attn2<128, 4>(value_bits, a, st);

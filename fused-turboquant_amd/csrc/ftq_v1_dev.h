@@ -80,7 +80,12 @@ bool v1_widths_ok(int kb, int vb, int flags);
 // The fp32 VALU decode (any head_dim of 64, 128, 256; every code width);
 // defined in ftq_v1_valu.hip.
 hipError_t v1_valu_launch(const V1Args& a, int d, int kb, int vb, int flags, hipStream_t st);
-// The same kernel over raw fp16 [K | V] slots (boundary layers; a.vrot = 0,
+// The matrix-core decode at float32-level products (head_dim 64 and 256, 2-4
+// bit codes, uniform V); defined in ftq_v1_split.hip.
+bool v1_split_takes(int d, int kb, int vb, int flags);
+hipError_t v1_split_launch(const V1Args& a, int d, int kb, int vb, hipStream_t st);
+int v1_split_resident(int d);
+// The VALU kernel over raw fp16 [K | V] slots (boundary layers; a.vrot = 0,
 // a.rot = null, a.qscale = scale * log2 e).
 hipError_t raw_valu_launch(const V1Args& a, int d, hipStream_t st);
 

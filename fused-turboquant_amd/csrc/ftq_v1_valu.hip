@@ -3,9 +3,10 @@
 // 42-442, every product and sum in fp32), for every slot format the store
 // writes -- head_dim 64, 128 or 256; K codes of 1, 2, 3, 4 or 8 bits or fp8
 // e4m3fn keys; V codes of 1, 2, 3, 4 or 8 bits, uniform or Lloyd-Max (4-bit).
-// The matrix-core kernels of ftq_v1.hip cover head_dim 128 with 2-4 bit codes
-// at f16 operand precision; this kernel is the path for everything else, and
-// for callers that ask for fp32 products.  The same kernel reads the raw fp16
+// The matrix-core kernels cover 2-4 bit codes (ftq_v1.hip: head_dim 128 at f16
+// operand precision; ftq_v1_split.hip: 64 and 256 at float32-level products);
+// this kernel is the path for everything else, and for callers that ask for
+// fp32 products.  The same kernel reads the raw fp16
 // [K | V] slots of the boundary layers (KB = VB = 16: no codes, no norms, no
 // rotation; reference triton_boundary_attn.py:28-219) at head_dim 64 and 256,
 // where ftq_raw.hip's matrix-core kernel covers 128.

@@ -392,8 +392,9 @@ def v1_decode_attention(query: torch.Tensor, kv_cache: torch.Tensor, block_table
     ``operands``: ``"f16"`` (default) runs head_dim 128 with 2-4 bit codes on
     the matrix-core kernels (f16 operands, fp32 accumulation); ``"fp32"``
     keeps every product in fp32 on the VALU, the reference's arithmetic.
-    Head dims 64 and 256, 1- and 8-bit codes and fp8 keys always take the
-    fp32 kernel.
+    Head dims 64 and 256 with 2-4 bit codes run on the matrix cores too, with
+    operands split so that the products are float32-level; 1- and 8-bit codes
+    and fp8 keys always take the fp32 kernel.
     """
     B, hq, d = query.shape
     _check_bits(d, key_bits, value_bits, key_fp8)

@@ -41,9 +41,9 @@ query block to its window.  The reference stores the window and attends the
 whole context (``:316``); logit soft-capping, which it also stores without
 applying (``:318``), is refused here.
 
-Head sizes 64, 128 and 256.  At 128 with 2-4 bit codes decode runs on the
-matrix-core kernels; every other head size and width (1-bit, 8-bit, fp8
-keys) runs the fp32 decode kernel.
+Head sizes 64, 128 and 256.  With 2-4 bit codes decode runs on the
+matrix-core kernels (64 and 256 at float32-level products); the other widths
+(1-bit, 8-bit, fp8 keys) run the fp32 decode kernel.
 
 Deferred prefill (``TURBOQUANT_DEFER_PREFILL=1``, TurboQuant layers; reference
 ``:331-332``, ``:673-686``, ``:1095-1277``): a prefill store of 1 < N <=
@@ -517,8 +517,8 @@ class FusedTurboQuantV1Impl(_ImplBase):
         n_q = q.shape[0]
         row = block_row.to(torch.int32)
         raw = self._is_raw
-        matrix = self.head_size == 128 and (raw or (2 <= self.key_bits <= 4 and 2 <= self.value_bits <= 4))
-        enough = n_q >= (_CHUNK_MIN_TOKENS if matrix else _CHUNK_MIN_TOKENS_VALU)
+        matrix = self.head_size == 128 if raw else 2 <= self.key_bits <= 4 and 2 <= self.value_bits <= 4
+        enough = n_q >= (_CHUNK_MIN_TOKENS if matrix else _CHUNK_MIN_TOKENS_FMA)
         if enough and not (self.v_lloyd_max and self.value_bits == 4):
             V1.v1_chunk_attention(q, kv_cache, row, past, None if raw or self.key_fp8 else st.centroids, self.key_bits,
                                   self.value_bits, self.scale, v_rotate=not raw and st.v_rotate,
@@ -558,9 +558,12 @@ _WINDOW_QUERY_BLOCK = 2048
 # pays one pass over the context whatever the chunk; the decode kernel pays one
 # per token.  Measured (bf16, K4V4, 8 kv heads, group 4; decode / chunk us):
 # d = 128, 8 tokens over 30000 positions 79 / 119, 16 tokens 132 / 118, over
-# 5120 44 / 44; d = 64, 4 tokens 85 / 91, 8 tokens 132 / 90.
+# 5120 44 / 44; d = 64 at 30000, 8 tokens 77 / 78, 16 tokens 128 / 76; d = 256
+# (4 kv heads, group 2) 8 tokens 90 / 109, 16 tokens 148 / 112.
 _CHUNK_MIN_TOKENS = 16
-_CHUNK_MIN_TOKENS_VALU = 8  # formats whose decode runs on the VALU
+# the other formats (1- and 8-bit codes, fp8 keys, raw slots at d = 64 / 256)
+# decode on the FMA kernel: d = 64, 8 tokens over 30000 positions 132 / 90
+_CHUNK_MIN_TOKENS_FMA = 8
 _GQA_KERNELS: Optional[bool] = None  # whether torch's fused SDPA kernels take grouped K/V here
 
 
