@@ -371,6 +371,44 @@ void lib_attention(const at::Tensor& query, const at::Tensor& codes_k, const std
   check_rc(ftq_lib_attention(&a, ws.data_ptr(), need, stream_of(query)));
 }
 
+// ---- steps of the HuggingFace attention forward ----
+
+// q [B, Hq, n, d], k [B, Hkv, n, d] (rows contiguous), cos / sin [B or 1, n, d]
+// -> the embedded q and k, [B, H, n, d] views of [B, n, H, d] storage
+std::tuple<at::Tensor, at::Tensor> rope(const at::Tensor& q, const at::Tensor& k, const at::Tensor& cos,
+                                        const at::Tensor& sin) {
+  on_device(q, "q");
+  on_device(k, "k");
+  on_device(cos, "cos");
+  on_device(sin, "sin");
+  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && q.size(0) == k.size(0) && q.size(2) == k.size(2) && q.size(3) == k.size(3),
+              "fused_tq: q and k must be [B, H, n, d]");
+  const int64_t B = q.size(0), n = q.size(2), d = q.size(3);
+  for (const at::Tensor* t : {&cos, &sin})
+    TORCH_CHECK(t->dim() == 3 && (t->size(0) == B || t->size(0) == 1) && t->size(1) == n && t->size(2) == d &&
+                    t->stride(2) == 1 && t->scalar_type() == q.scalar_type(),
+                "fused_tq: cos and sin must be [B or 1, n, d] of q's type");
+  TORCH_CHECK(q.stride(3) == 1 && k.stride(3) == 1 && q.scalar_type() == k.scalar_type(), "fused_tq: rows must be contiguous");
+  const c10::DeviceGuard g(q.device());
+  at::Tensor qo = at::empty({B, n, q.size(1), d}, q.options()), ko = at::empty({B, n, k.size(1), d}, k.options());
+  if (qo.numel() > 0 && ko.numel() > 0)
+    check_rc(ftq_rope(q.data_ptr(), qo.data_ptr(), q.stride(0), q.stride(1), q.stride(2), (int)q.size(1), k.data_ptr(),
+                      ko.data_ptr(), k.stride(0), k.stride(1), k.stride(2), (int)k.size(1), cos.data_ptr(),
+                      cos.size(0) == 1 ? 0 : cos.stride(0), cos.stride(1), sin.data_ptr(),
+                      sin.size(0) == 1 ? 0 : sin.stride(0), sin.stride(1), dt(q), (int)B, (int)n, (int)d, stream_of(q)));
+  return {qo.transpose(1, 2), ko.transpose(1, 2)};
+}
+
+at::Tensor append_slots(at::Tensor& lens, int64_t n, int64_t capacity) {
+  contig(lens, "lens");
+  TORCH_CHECK(lens.scalar_type() == at::kInt && n >= 0 && n <= INT32_MAX, "fused_tq: lens must be int32");
+  const c10::DeviceGuard g(lens.device());
+  at::Tensor slots = at::empty({lens.numel() * n}, lens.options().dtype(at::kLong));
+  check_rc(ftq_append_slots(lens.data_ptr<int32_t>(), slots.data_ptr<int64_t>(), (int)lens.numel(), (int)n, capacity,
+                            stream_of(lens)));
+  return slots;
+}
+
 // ---- raw fp16 slots (boundary layers) -------------------------------------
 
 void raw_store(const at::Tensor& key, const at::Tensor& value, at::Tensor& kv_cache, const at::Tensor& slot_mapping) {
@@ -437,6 +475,8 @@ TORCH_LIBRARY(fused_tq, m) {
         "Tensor? block_table, Tensor lens, Tensor? new_key, Tensor? new_value, Tensor k_signs, Tensor v_signs, "
         "Tensor k_levels, Tensor v_levels, int bits_k, int bits_v, int max_len, float scale, int window, int sinks, "
         "bool precise, Tensor(a!) out) -> ()");
+  m.def("rope(Tensor q, Tensor k, Tensor cos, Tensor sin) -> (Tensor, Tensor)");
+  m.def("append_slots(Tensor(a!) lens, int n, int capacity) -> Tensor");
   m.def("raw_store(Tensor key, Tensor value, Tensor(a!) kv_cache, Tensor slot_mapping) -> ()");
   m.def("raw_decode_attention(Tensor query, Tensor kv_cache, Tensor block_table, Tensor seq_lens, "
         "Tensor? kv_start, float scale, int num_splits, Tensor(a!) workspace, Tensor(b!) out, "
@@ -454,6 +494,8 @@ TORCH_LIBRARY_IMPL(fused_tq, CUDA, m) {
   m.impl("v1_decode_attention", &v1_decode_attention);
   m.impl("v1_chunk_attention", &v1_chunk_attention);
   m.impl("lib_attention", &lib_attention);
+  m.impl("rope", &rope);
+  m.impl("append_slots", &append_slots);
   m.impl("raw_store", &raw_store);
   m.impl("raw_decode_attention", &raw_decode_attention);
 }

@@ -49,6 +49,14 @@ def _register_fakes() -> None:
     def _rht(x, signs, inverse, out_dtype):
         return x.new_empty(x.shape, dtype=out_dtype)
 
+    @torch.library.register_fake(lib + "rope")
+    def _rope(q, k, cos, sin):
+        return tuple(x.new_empty((x.shape[0], x.shape[2], x.shape[1], x.shape[3])).transpose(1, 2) for x in (q, k))
+
+    @torch.library.register_fake(lib + "append_slots")
+    def _append_slots(lens, n, capacity):
+        return lens.new_empty((lens.numel() * n,), dtype=torch.int64)
+
     # operators that only write their (a!) arguments
     for name in ("paged_store", "paged_decode_attention", "v1_store", "v1_decode_attention",
                  "v1_chunk_attention", "lib_attention", "raw_store", "raw_decode_attention"):

@@ -46,6 +46,7 @@ import torch
 import torch.nn.functional as F
 from transformers import DynamicCache
 
+from .. import _ops
 from .. import paged as P
 from ..core.quantizer import CompressedTensor, TurboQuantMSE
 
@@ -92,18 +93,16 @@ class _LayerPages:
             fresh.view(self.B, new_cap, *shape[1:])[:, :self.cap] = self.kv_cache.view(self.B, self.cap, *shape[1:])
         self.kv_cache = fresh
         self.cap = new_cap
-        self.block_table = (torch.arange(self.B, device=self.device, dtype=torch.int32).view(-1, 1) * new_cap
-                            + torch.arange(new_cap, device=self.device, dtype=torch.int32).view(1, -1))
+        self.block_table = torch.arange(self.B * new_cap, device=self.device, dtype=torch.int32).view(self.B, new_cap)
 
     def append(self, key: torch.Tensor, value: torch.Tensor, keep: Optional[torch.Tensor]) -> None:
         """key/value [B, Hkv, q, d]; keep [B, q] bool (None = every token)."""
         B, hkv, q, d = key.shape
         if keep is None:
             self._ensure(max(self.lens) + q)
-            # slots computed on the device: no host round trip per decode step
-            base = torch.arange(B, device=self.device, dtype=torch.int64) * (self.cap * _PAGE)
-            slot_t = (base.view(-1, 1) + self.lens_dev.view(-1, 1).to(torch.int64)
-                      + torch.arange(q, device=self.device, dtype=torch.int64).view(1, -1)).reshape(-1)
+            # slots computed (and the lengths advanced) on the device: no host
+            # round trip per decode step
+            slot_t = _ops.ops().append_slots(self.lens_dev, q, self.cap * _PAGE)
             self.lens = [L + q for L in self.lens]
             new_lens = None
         else:
@@ -125,9 +124,7 @@ class _LayerPages:
         k = key.permute(0, 2, 1, 3).reshape(B * q, hkv, d)
         v = value.permute(0, 2, 1, 3).reshape(B * q, hkv, d)
         P.paged_store(k, v, self.kv_cache, slot_t, self.k_tq, self.v_tq)
-        if new_lens is None:
-            self.lens_dev.add_(q)
-        else:
+        if new_lens is not None:
             self.lens_dev.copy_(new_lens)
 
     def flat(self):
@@ -332,7 +329,7 @@ class CompressedKVCache(DynamicCache):
     def _fused_attention(lp, query: torch.Tensor) -> bool:
         """Whether the library-format attention kernels take this layer and query."""
         hq, d = query.shape[1], query.shape[-1]
-        return (d == lp.d and d in P.LIB_ATTENTION_DIMS and hq % lp.hkv == 0 and hq // lp.hkv <= 16
+        return (not _needs_grad(query) and d == lp.d and d in P.LIB_ATTENTION_DIMS and hq % lp.hkv == 0 and hq // lp.hkv <= 16
                 and lp.B * lp.hkv <= 65535 and query.dtype in (torch.float32, torch.float16, torch.bfloat16))
 
     @staticmethod
@@ -349,8 +346,8 @@ class CompressedKVCache(DynamicCache):
         compressed past and the step's own tokens, causal.  None where the
         kernels do not take the layer."""
         lp = self._pages[layer_idx]
-        if not self._fused_attention(lp, query) or key.dtype != value.dtype or key.dtype not in (
-                torch.float32, torch.float16, torch.bfloat16):
+        if not self._fused_attention(lp, query) or _needs_grad(key, value) or key.dtype != value.dtype \
+                or key.dtype not in (torch.float32, torch.float16, torch.bfloat16):
             return None
         return self._lib_attention(lp, query, scale, new_kv=(key, value), window=sliding_window)
 
@@ -372,6 +369,24 @@ def _rotate_half(x):
 def _apply_rotary_pos_emb(q, k, cos, sin):
     cos, sin = cos.unsqueeze(1), sin.unsqueeze(1)
     return (q * cos) + (_rotate_half(q) * sin), (k * cos) + (_rotate_half(k) * sin)
+
+
+def _rope_fused(q, k, cos, sin) -> bool:
+    """Whether the rotary embedding of q / k [B, H, n, d] runs as one kernel
+    (the same roundings as the torch expression): device tensors of one type,
+    full-width cos / sin, aligned rows, nothing to differentiate."""
+    d = q.shape[-1]
+    return (q.is_cuda and q.dtype in (torch.float32, torch.float16, torch.bfloat16) and d % 16 == 0
+            and k.dtype == q.dtype and cos.dtype == q.dtype and sin.dtype == q.dtype
+            and cos.dim() == 3 and sin.shape == cos.shape and tuple(cos.shape[1:]) == (q.shape[2], d)
+            and cos.shape[0] in (1, q.shape[0]) and k.shape[0] == q.shape[0] and k.shape[2:] == q.shape[2:]
+            and not _needs_grad(q, k, cos, sin)
+            and all(t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1])
+                    for t in (q, k, cos, sin)))
+
+
+def _needs_grad(*tensors) -> bool:
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
 
 
 def _repeat_kv(x: torch.Tensor, n_rep: int) -> torch.Tensor:
@@ -524,7 +539,10 @@ def make_fused_attention_forward(attn_module, cache: CompressedKVCache, quantize
             v = v_norm(v)
         if position_embeddings is not None:
             cos, sin = position_embeddings
-            q, k = _apply_rotary_pos_emb(q, k, cos, sin)
+            if _rope_fused(q, k, cos, sin):
+                q, k = _ops.ops().rope(q, k, cos, sin)
+            else:
+                q, k = _apply_rotary_pos_emb(q, k, cos, sin)
 
         lens_before = cache.seq_lens(layer_idx)  # per sequence, before this chunk is stored
         had_past = bool(lens_before) and max(lens_before) > 0

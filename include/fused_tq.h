@@ -452,6 +452,20 @@ int64_t ftq_lib_attention_workspace_bytes(int batch, int n_query, int num_q_head
 int ftq_lib_attention(const ftq_lib_attention_args* args, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * Rotary embedding of a step's queries and keys, x cos + rotate_half(x) sin
+ * with the products and the sum rounded to the type (the torch expression of
+ * reference hf/fused_cache.py:540-560); rows [batch][heads][tokens][d] by
+ * element strides (multiples of 8), outputs contiguous [batch][tokens][heads][d];
+ * cos / sin [batch or 1][tokens][d] (batch stride 0 for one).
+ */
+int ftq_rope(const void* q, void* q_out, int64_t q_batch, int64_t q_head, int64_t q_tok, int num_q_heads,
+             const void* k, void* k_out, int64_t k_batch, int64_t k_head, int64_t k_tok, int num_kv_heads,
+             const void* cos, int64_t cos_batch, int64_t cos_tok, const void* sin, int64_t sin_batch,
+             int64_t sin_tok, int dtype, int batch, int tokens, int d, void* stream);
+/* slots[b * n + i] = b * capacity + lens[b] + i, then lens[b] += n (batch sequences). */
+int ftq_append_slots(int32_t* lens, int64_t* slots, int batch, int n, int64_t capacity, void* stream);
+
+/*
  * Store n_tokens x num_kv_heads K/V vectors ([n][Hkv][d], dtype) as fp16
  * (round to nearest even) into their raw slots; slot_mapping[i] < 0 skips
  * token i (and a slot past the cache is skipped too).  Replaces _store_raw_kv

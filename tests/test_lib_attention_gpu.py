@@ -120,3 +120,30 @@ def test_large_values_stay_finite(cuda):
     cache.store_compressed_kv(k.to(dt).to(cuda), v.to(dt).to(cuda), 0)
     got = cache.chunk_attention(q.to(dt).to(cuda), k.to(dt).to(cuda), v.to(dt).to(cuda), 0, 0.125)
     assert torch.isfinite(got).all() and got.abs().max() > 1000
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,hq,hkv,n,d,cb", [(2, 8, 2, 5, 64, 2), (1, 4, 4, 1, 128, 1), (3, 7, 1, 33, 256, 1)])
+def test_rope_kernel_is_the_torch_expression(cuda, dtype, B, hq, hkv, n, d, cb):
+    """Bit for bit, on transposed views, with one or B sets of angles."""
+    from fused_turboquant.hf import fused_cache as F
+    from fused_turboquant import _ops
+    g = torch.Generator().manual_seed(n)
+    q = torch.randn(B, n, hq, d, generator=g).to(dtype).to(cuda).transpose(1, 2)
+    k = torch.randn(B, n, hkv, d, generator=g).to(dtype).to(cuda).transpose(1, 2)
+    ang = torch.randn(cb, n, d, generator=g) * 3
+    cos, sin = ang.cos().to(dtype).to(cuda), ang.sin().to(dtype).to(cuda)
+    assert F._rope_fused(q, k, cos, sin)
+    got, want = _ops.ops().rope(q, k, cos, sin), F._apply_rotary_pos_emb(q, k, cos, sin)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and a.transpose(1, 2).is_contiguous() and torch.equal(a, b)
+    assert not F._rope_fused(q, k, cos[..., : d // 2], sin[..., : d // 2])  # partial rotary: the torch expression
+    assert not F._rope_fused(q.requires_grad_(), k, cos, sin)
+
+
+def test_append_slots(cuda):
+    from fused_turboquant import _ops
+    lens = torch.tensor([0, 7, 300], dtype=torch.int32, device=cuda)
+    got = _ops.ops().append_slots(lens, 260, 1000)
+    want = torch.cat([b * 1000 + n + torch.arange(260) for b, n in enumerate((0, 7, 300))])
+    assert torch.equal(got.cpu(), want) and lens.tolist() == [260, 267, 560]
