@@ -24,11 +24,24 @@
 //      from the score registers into the P.V operand without a shuffle
 //   Q  [16-column tile][s][part][lane]: column m, dims 32 s + 8 g + j
 // A column is a (query row, head of the kv head's group) pair, row-major.
+//
+// Bound by the matrix cores and the softmax beside them: the hi + lo query and
+// weights double the products, and 1024 query tokens over 6144 positions (32
+// heads over 8 at d = 128, 4-bit) run 189 GFLOP of them in 182 us, 1.04
+// PFLOP/s where a large library product in the same type reaches 1.33.  Before
+// that: 231 us with the tiles staged through registers and the masks of the
+// edges in every tile.  The tiles now go to LDS directly (17 registers free,
+// which is what lets the low parts and the sums run under the high parts'
+// products), and only the tiles at the edges of the causal range or the window
+// carry masks, in a copy of the loop.  d = 64: 190 -> 157 us; d = 256 (8 heads
+// over 4): 197 -> 155; d = 128 with 8-bit K and V: 329 -> 223.
 #pragma once
 
 #include "ftq_attn_dev.h"
 #include "ftq_merge.h"
 #include "ftq_v1_dev.h"
+
+#include <type_traits>
 
 namespace ftq {
 
@@ -74,6 +87,16 @@ __device__ __forceinline__ float fwht_pair32(float x, bool upper) {
   return upper ? a - b : a + b;
 }
 
+// 16 (4) bytes of each lane to base + 16 (4) * lane in LDS; base is the wave's
+__device__ __forceinline__ void lds_load16(const void* src, void* base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)base, 16, 0, 0);
+}
+__device__ __forceinline__ void lds_load4(const void* src, void* base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)base, 4, 0, 0);
+}
+
 // f16 pair of two floats, each rounded to nearest (v_cvt_pk_f16_f32)
 __device__ __forceinline__ uint32_t pk_f16(float a, float b) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -90,14 +113,14 @@ __device__ __forceinline__ float f16_rest(float x, uint32_t w, int half) {
 // fragments as hi + lo (Lloyd-Max V at that precision); ZM: V has a per-token
 // minimum, and positions may be hidden by their bias.
 template <int D, int NH, bool KHL, bool VHL, bool ZM>
-__global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
+__global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const ChunkAttn a) {
   using C = ChunkGeo<D, KHL>;
   constexpr int CT = C::CT, TK = C::TK, NS = C::NS, NB = C::NB, NT = C::NT, NP = C::NP;
   constexpr int KP = KHL ? 2 : 1;
   constexpr int VP = VHL ? 2 : 1;
   static_assert(!VHL || KHL, "V hi + lo goes with K hi + lo");
   constexpr int KU = NT * NS * KP * 64, VU = NP * NB * VP * 64;  // 16-byte units of a tile
-  constexpr int KT = KU / 256 / KP, VT = VU / 256 / VP;
+  static_assert(KU % 256 == 0 && VU % 256 == 0 && 4 * TK % 64 == 0, "whole waves fetch a tile");
   __shared__ u32x4 kb[2][KU];
   __shared__ u32x4 vb[2][VU];
   __shared__ __attribute__((aligned(16))) float tb[2][4][TK];
@@ -117,16 +140,15 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
   const int c0 = blk * C::COLS;
   const int r_lo = c0 / a.G, r_hi = (min(c0 + C::COLS, ncols) - 1) / a.G;
   const int wc0 = c0 + wave * 16 * CT;
-  const int wr_lo = min(wc0 / a.G, a.nq - 1), wr_hi = min((wc0 + 16 * CT - 1) / a.G, a.nq - 1);
   const int first = a.window > 0 ? max(0, past + r_lo + 1 - a.window) : 0;
   const int t0 = max(first, a.seg0) / TK;
   const int t1 = (min(past + r_hi + 1, a.seg1) + TK - 1) / TK;
   const int nt = t1 > t0 ? t1 - t0 : 0;
   const int per = (nt + a.splits - 1) / a.splits;
   const int tb0 = t0 + split * per, tb1 = min(tb0 + per, t1);
-  // positions every / any row of the wave attends
-  const int w_all = past + wr_lo + 1;                                     // below: in every row's causal range
-  const int w_from = a.window > 0 ? max(0, past + wr_hi + 1 - a.window) : 0;  // from: in every row's window
+  // positions that every row of the workgroup attends: [w_from, w_all)
+  const int w_all = past + r_lo + 1;
+  const int w_from = a.window > 0 ? max(0, past + r_hi + 1 - a.window) : 0;
   int lim[CT], lo[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
@@ -139,42 +161,18 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
   const u32x4* vf = a.vf + (int64_t)kvh * a.vstride;
   const float* tk = a.tok + (int64_t)kvh * a.tstride;
   const int tseg = a.seg0 / TK;
-  u32x4 rk[KT], rl[KHL ? KT : 1], rv[VT], rw[VHL ? VT : 1];
-  float rt = 0.f;
-  auto fetch = [&](int t) __attribute__((always_inline)) {
+  // a tile's fragments go straight to LDS (fragment order is lane order)
+  auto fetch = [&](int t, int p) __attribute__((always_inline)) {
     const u32x4* pk = kf + (int64_t)(t - tseg) * KU + tid;
     const u32x4* pv = vf + (int64_t)(t - tseg) * VU + tid;
 #pragma unroll
-    for (int j = 0; j < KT; ++j) rk[j] = pk[256 * j];
-    if constexpr (KHL) {
+    for (int j = 0; j < KU / 256; ++j) lds_load16(pk + 256 * j, &kb[p][256 * j + 64 * wave]);
 #pragma unroll
-      for (int j = 0; j < KT; ++j) rl[j] = pk[256 * (KT + j)];
-    }
-#pragma unroll
-    for (int j = 0; j < VT; ++j) rv[j] = pv[256 * j];
-    if constexpr (VHL) {
-#pragma unroll
-      for (int j = 0; j < VT; ++j) rw[j] = pv[256 * (VT + j)];
-    }
-    if (tid < 4 * TK) rt = tk[(int64_t)(t - tseg) * 4 * TK + tid];
-  };
-  auto commit = [&](int p) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < KT; ++j) kb[p][tid + 256 * j] = rk[j];
-    if constexpr (KHL) {
-#pragma unroll
-      for (int j = 0; j < KT; ++j) kb[p][tid + 256 * (KT + j)] = rl[j];
-    }
-#pragma unroll
-    for (int j = 0; j < VT; ++j) vb[p][tid + 256 * j] = rv[j];
-    if constexpr (VHL) {
-#pragma unroll
-      for (int j = 0; j < VT; ++j) vb[p][tid + 256 * (VT + j)] = rw[j];
-    }
-    if (tid < 4 * TK) (&tb[p][0][0])[tid] = rt;
+    for (int j = 0; j < VU / 256; ++j) lds_load16(pv + 256 * j, &vb[p][256 * j + 64 * wave]);
+    if (wave < 4 * TK / 64) lds_load4(tk + (int64_t)(t - tseg) * 4 * TK + tid, &tb[p][0][0] + 64 * wave);
   };
 
-  if (tb0 < tb1) fetch(tb0);
+  if (tb0 < tb1) fetch(tb0, 0);
   // the query operands of the wave's columns
   half8 qh[CT][NS], ql[NH == 2 ? CT : 1][NH == 2 ? NS : 1];
   float qs[CT];
@@ -201,7 +199,9 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
     for (int b = 0; b < NB; ++b) acc[ct][b] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
-  auto process = [&](int t, int p) __attribute__((always_inline)) {
+  // edge: the tile has positions that some row of the workgroup does not attend
+  auto process = [&](int t, int p, bool more, auto edge_c) __attribute__((always_inline)) {
+    constexpr bool edge = decltype(edge_c)::value;
     floatx4 s[NT][CT];
 #pragma unroll
     for (int k = 0; k < NT; ++k)
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
         }
       }
     }
-    constexpr bool VEARLY = !VHL && NP * NB <= 8;
+    constexpr bool VEARLY = !VHL;
     half8 xv[VEARLY ? NP * NB : 1];
     if constexpr (VEARLY) {
       __builtin_amdgcn_sched_barrier(0);
@@ -268,27 +268,32 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
       for (int i = 0; i < NP * NB; ++i) xv[i] = __builtin_bit_cast(half8, vb[p][i * 64 + lane]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const bool edge = t * TK + TK > w_all || t * TK < w_from;  // wave-uniform
+    float tf[NT][4][4];  // the tile's factors of this lane's tokens: K factor, bias, V factor, V minimum
+#pragma unroll
+    for (int k = 0; k < NT; ++k)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        if (!ZM && (f & 1)) continue;
+        const float4 x = *reinterpret_cast<const float4*>(&tb[p][f][16 * k + 4 * g]);
+        tf[k][f][0] = x.x; tf[k][f][1] = x.y; tf[k][f][2] = x.z; tf[k][f][3] = x.w;
+      }
+    // The next tile is requested here: behind the reads of this one, or the
+    // compiler, which does not tell the two buffers apart, waits for it before
+    // each of them.
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) fetch(t + 1, p ^ 1);
     // scores: x K factor (and the column's), + bias; masked on the edges
 #pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      const float4 f4 = *reinterpret_cast<const float4*>(&tb[p][0][16 * k + 4 * g]);
-      const float fa[4] = {f4.x, f4.y, f4.z, f4.w};
-      float ba[4] = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (ZM) {
-        const float4 b4 = *reinterpret_cast<const float4*>(&tb[p][1][16 * k + 4 * g]);
-        ba[0] = b4.x; ba[1] = b4.y; ba[2] = b4.z; ba[3] = b4.w;
-      }
+    for (int k = 0; k < NT; ++k)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float y = s[k][ct][i];
           if constexpr (KHL) y = (y + sl[k][ct][i]) * qs[ct];
-          s[k][ct][i] = ZM ? __builtin_fmaf(y, fa[i], ba[i]) : y * fa[i];
+          s[k][ct][i] = ZM ? __builtin_fmaf(y, tf[k][0][i], tf[k][1][i]) : y * tf[k][0][i];
         }
-    }
-    if (edge) {
+    if constexpr (edge) {
 #pragma unroll
       for (int k = 0; k < NT; ++k)
 #pragma unroll
@@ -321,78 +326,84 @@ __global__ __launch_bounds__(256, 2) void chunk_attn_kernel(const ChunkAttn a) {
     u32x4 ph[NP][CT], pl[NH == 2 ? NP : 1][NH == 2 ? CT : 1];
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
-      const float4 v4 = *reinterpret_cast<const float4*>(&tb[p][2][16 * k + 4 * g]);
-      const float va[4] = {v4.x, v4.y, v4.z, v4.w};
-      float za[4] = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (ZM) {
-        const float4 z4 = *reinterpret_cast<const float4*>(&tb[p][3][16 * k + 4 * g]);
-        za[0] = z4.x; za[1] = z4.y; za[2] = z4.z; za[3] = z4.w;
-      }
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
         float w[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+          const bool hid = edge && s[k][ct][i] == -INFINITY;  // its factors may be infinite or NaN
           const float e = __builtin_amdgcn_exp2f(s[k][ct][i] - m_run[ct]);
-          l_run[ct] += e;
-          float vv = va[i], zz = za[i];
-          if (edge) {  // a hidden position's factors may be infinite or NaN
-            const bool hid = s[k][ct][i] == -INFINITY;
-            vv = hid ? 0.f : vv;
-            zz = hid ? 0.f : zz;
-          }
-          if constexpr (ZM) z_run[ct] = __builtin_fmaf(e, zz, z_run[ct]);
-          w[i] = e * vv;
+          w[i] = e * (hid ? 0.f : tf[k][2][i]);
+          s[k][ct][i] = hid ? -1.f : e;
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const uint32_t hi = pk_f16(w[2 * h], w[2 * h + 1]);
-          ph[k >> 1][ct][2 * (k & 1) + h] = hi;
-          if constexpr (NH == 2)
-            pl[k >> 1][ct][2 * (k & 1) + h] = pk_f16(f16_rest(w[2 * h], hi, 0), f16_rest(w[2 * h + 1], hi, 1));
+        for (int h = 0; h < 2; ++h) ph[k >> 1][ct][2 * (k & 1) + h] = pk_f16(w[2 * h], w[2 * h + 1]);
+      }
+    }
+    // what the high parts' products leave time for: the low parts and the sums
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        float r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool hid = edge && s[k][ct][i] < 0.f;
+          const float e = hid ? 0.f : s[k][ct][i];
+          l_run[ct] += e;
+          if constexpr (ZM) z_run[ct] = __builtin_fmaf(e, hid ? 0.f : tf[k][3][i], z_run[ct]);
+          const half2_t hi = __builtin_bit_cast(half2_t, (uint32_t)ph[k >> 1][ct][2 * (k & 1) + (i >> 1)]);
+          if constexpr (NH == 2) r[i] = __builtin_fmaf(e, hid ? 0.f : tf[k][2][i], -(float)hi[i & 1]);
+        }
+        if constexpr (NH == 2) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) pl[k >> 1][ct][2 * (k & 1) + h] = pk_f16(r[2 * h], r[2 * h + 1]);
         }
       }
     }
 #pragma unroll
-    for (int k = 0; k < NP; ++k)
+    for (int part = VHL ? -1 : 0; part < NH; ++part)
 #pragma unroll
-      for (int b0 = 0; b0 < NB; b0 += 2) {
-        half8 x[2], z[2];
+      for (int k = 0; k < NP; ++k)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          if constexpr (VEARLY) x[b] = xv[k * NB + b0 + b];
-          else x[b] = __builtin_bit_cast(half8, vb[p][((k * NB + b0 + b) * VP) * 64 + lane]);
-          if constexpr (VHL) z[b] = __builtin_bit_cast(half8, vb[p][((k * NB + b0 + b) * VP + 1) * 64 + lane]);
-        }
+        for (int b = 0; b < NB; ++b) {
+          half8 x;
+          if constexpr (VEARLY) x = xv[k * NB + b];
+          else x = __builtin_bit_cast(half8, vb[p][((k * NB + b) * VP + (part < 0)) * 64 + lane]);
 #pragma unroll
-        for (int part = VHL ? -1 : 0; part < NH; ++part)
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-              const half8 w = part < 0 ? z[b] : x[b];
-              u32x4 pw = ph[k][ct];
-              if constexpr (NH == 2) {
-                if (part == 1) pw = pl[k][ct];
-              }
-              acc[ct][b0 + b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, __builtin_bit_cast(half8, pw), acc[ct][b0 + b], 0, 0, 0);
+          for (int ct = 0; ct < CT; ++ct) {
+            u32x4 pw = ph[k][ct];
+            if constexpr (NH == 2) {
+              if (part == 1) pw = pl[k][ct];
             }
-      }
+            acc[ct][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8, pw), acc[ct][b], 0, 0, 0);
+          }
+        }
+    // the sums are done in this block, under the matrix products
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) asm volatile("" : "+v"(l_run[ct]), "+v"(z_run[ct]));
+
   };
 
   // one barrier a tile: a buffer is refilled in the iteration after its
-  // readers passed the barrier that ended theirs
-  if (tb0 < tb1) commit(0);
-  // the query operands have arrived before the loop (vmcnt 0), or the loop
-  // would wait for them behind each next tile's loads
+  // readers passed the barrier that ended theirs, and has arrived (vmcnt 0)
+  // before the barrier that precedes its readers
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
-  int p = 0;
-  for (int t = tb0; t < tb1; ++t, p ^= 1) {
-    if (t + 1 < tb1) fetch(t + 1);
-    process(t, p);
-    if (t + 1 < tb1) commit(p ^ 1);
-    __syncthreads();
+  // tiles that some row of the workgroup attends in part, whole tiles, and again the former
+  const int ta = min(max((w_from + TK - 1) / TK, tb0), tb1), tz = max(min(w_all / TK, tb1), ta);
+  int p = 0, t = tb0;
+  auto tiles = [&](int end, auto edge_c) __attribute__((always_inline)) {
+    for (; t < end; ++t, p ^= 1) {
+      process(t, p, t + 1 < tb1, edge_c);
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+    }
+  };
+#pragma unroll 1
+  for (int part = 0; part < 2; ++part) {
+    tiles(part == 0 ? ta : tb1, std::true_type{});
+    if (part == 0) tiles(tz, std::false_type{});
   }
 
   // ---- output: lane (n, g) holds dims 16 b + 4 g + i of column n ----
