@@ -44,6 +44,7 @@ from typing import Optional
 
 import torch
 import torch.nn.functional as F
+from torch.autograd.forward_ad import unpack_dual
 from transformers import DynamicCache
 
 from .. import _ops
@@ -386,7 +387,9 @@ def _rope_fused(q, k, cos, sin) -> bool:
 
 
 def _needs_grad(*tensors) -> bool:
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+    """Whether a derivative, backward or forward mode, has to pass the tensors."""
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+            or any(unpack_dual(t).tangent is not None for t in tensors))
 
 
 def _repeat_kv(x: torch.Tensor, n_rep: int) -> torch.Tensor:
