@@ -1514,18 +1514,19 @@ static hipError_t launch_attn_valu2(int bv, const AttnArgs& a, hipStream_t st) {
 }
 
 // Splits of a grid that does not fill the GPU: up to one workgroup per CU (256)
-// while each split keeps about 64 positions, and none where that saves less
-// than the merge costs.  A workgroup alone on its CU walks its tiles at their
-// latency (1-1.6 us each), so the longest walk sets the time.  Measured (us at
-// the earlier count of 8 tiles per wave / this one): paged d = 128, 1 x 8 units,
-// 1200 positions 15 / 10, 5000 19 / 11, 10000 19 / 12; 4 x 8 units, 1200 15 /
-// 11, 5000 20 / 15; 16 x 8, 2500 equal; d = 256, 1 x 8, 5000 26 / 14; v1 slots
-// the same within 10%.  250 positions: 1 split 8.5-9, 4 splits 9-9.2.
-int small_grid_splits(int64_t units, int64_t positions, int64_t from) {
+// while each split keeps about 64 positions.  A workgroup alone on its CU walks
+// its tiles at their latency (1-1.6 us each), so the longest walk sets the
+// time.  Measured (us at the count of 8 tiles per wave / this one): paged d =
+// 128, 1 x 8 units, 5000 positions 19 / 11, 10000 19 / 12; 4 x 8 units, 5000 20
+// / 15; 16 x 8, 2500 equal; d = 256, 1 x 8, 5000 26 / 14; v1 slots the same
+// within 10%.  From 2048 positions, where the other count splits too: below, a
+// second launch and a workspace would be added, which cost the host 2.5-3 us
+// (decode steps through the HuggingFace cache 15.0 -> 17.5, vLLM layers 38.5
+// -> 41), while the one launch's 10-25 us run in the shadow of that host time.
+int small_grid_splits(int64_t units, int64_t positions) {
   if (units < 1) units = 1;
-  if (positions < from) return 1;
-  const int64_t s = std::min<int64_t>(std::min<int64_t>(256 / units, (positions + 63) / 64), 64);
-  return s < 2 || (s < 4 && positions < 1000) ? 1 : (int)s;
+  if (positions < 2048) return 1;
+  return (int)std::max<int64_t>(std::min<int64_t>(std::min<int64_t>(256 / units, (positions + 63) / 64), 64), 1);
 }
 
 int auto_splits(int batch, int hkv, int seq_hint, int target_wgs) {
@@ -1535,7 +1536,7 @@ int auto_splits(int batch, int hkv, int seq_hint, int target_wgs) {
   int s = (int)std::min<int64_t>((target_wgs + units - 1) / units, 64);
   const int max_by_len = seq_hint / (32 * 4 * 8);
   if (s > max_by_len) s = max_by_len;
-  s = std::max(s, small_grid_splits(units, seq_hint, 400));
+  s = std::max(s, small_grid_splits(units, seq_hint));
   if (s < 1) s = 1;
   if (s > 64) s = 64;
   return s;

@@ -1375,7 +1375,7 @@ static hipError_t v1_launch_attn2(int vb, const V1Args& a, hipStream_t st) {
 }
 
 int auto_splits(int batch, int hkv, int seq_hint, int target_wgs);
-int small_grid_splits(int64_t units, int64_t positions, int64_t from);
+int small_grid_splits(int64_t units, int64_t positions);
 
 }  // namespace ftq
 
@@ -1480,10 +1480,9 @@ extern "C" int ftq_v1_choose_splits(int batch, int num_q_heads, int num_kv_heads
   // faster than 1; 448 and 512 units at K3 V3, 1 split best (two splits
   // would need a second round); K4 V2 at 448 and 512, 2 splits 1-11%
   // faster; 4 x 8 units at 64K-128K, K4 V2, 32 splits.  No more splits than
-  // leave 8 tiles per wave, and at most 64 -- or, from 1024 positions (400 on
-  // the split-operand kernel), what a grid that does not fill the GPU takes
-  // (small_grid_splits): 1 x 8 units, K4 V4, group 4, 1200 positions 17 -> 10
-  // us, 5000 19 -> 12; d = 64 the same, d = 256 21 -> 13 and 38 -> 17.
+  // leave 8 tiles per wave, and at most 64 -- or what a grid that does not
+  // fill the GPU takes (small_grid_splits): 1 x 8 units, K4 V4, group 4, 5000
+  // positions 19 -> 12 us; d = 64 the same, d = 256 38 -> 17.
   const int group = num_q_heads / num_kv_heads;
   const bool lloyd = value_bits == 4 && (v_flags & V1F_VLM) != 0;
   int cap;
@@ -1495,7 +1494,7 @@ extern "C" int ftq_v1_choose_splits(int batch, int num_q_heads, int num_kv_heads
   int64_t s = cap / units;
   const int64_t by_len = max_seq_len / (32 * 4 * 8);
   if (s > by_len) s = by_len;
-  s = std::max<int64_t>(s, small_grid_splits(units, max_seq_len, split_ops ? 400 : 1024));
+  s = std::max<int64_t>(s, small_grid_splits(units, max_seq_len));
   if (s > 64) s = 64;
   return s < 1 ? 1 : (int)s;
 }
