@@ -417,7 +417,11 @@ hipError_t lib_launch(const LibPlan& p, LibSource s, const void* q, int qt, int6
     chunk_gather_lib_kernel<D, PREC><<<dim3((a.seg1 - a.seg0) / 32, units), dim3(256), 0, st>>>(
         s, hkv, a.seg0, kf, p.kstride, vf, p.vstride, tok, p.tstride);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    chunk_attn_kernel<D, NH, PREC, PREC, PREC><<<dim3((unsigned)(units * (p.colpad / p.cols)), p.splits), dim3(256), 0, st>>>(a);
+    // A decode step hides positions by their bias (ZM); a multi-token step's
+    // f16 form has none to hide below its causal limits and skips the bias.
+    const dim3 agrid((unsigned)(units * (p.colpad / p.cols)), p.splits);
+    if (decode || PREC) chunk_attn_kernel<D, NH, PREC, PREC, true><<<agrid, dim3(256), 0, st>>>(a);
+    else chunk_attn_kernel<D, NH, PREC, PREC, PREC><<<agrid, dim3(256), 0, st>>>(a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (direct) return hipSuccess;

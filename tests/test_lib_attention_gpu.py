@@ -147,3 +147,37 @@ def test_append_slots(cuda):
     got = _ops.ops().append_slots(lens, 260, 1000)
     want = torch.cat([b * 1000 + n + torch.arange(260) for b, n in enumerate((0, 7, 300))])
     assert torch.equal(got.cpu(), want) and lens.tolist() == [260, 267, 560]
+
+
+def _lib(cache, q, window=None, sinks=0, precise=None, new_kv=None, lens=None, max_len=None):
+    """``paged.lib_attention`` on a cache's layer, query [B, Hq, n, d]."""
+    from fused_turboquant import paged as P
+    lp = cache._pages[0]
+    src = dict(pages=(lp.kv_cache, lp.block_table)) if lp.d in (128, 256) else dict(flat=(lp.kp, lp.kn, lp.vp, lp.vn))
+    return P.lib_attention(q, lp.lens_dev if lens is None else lens, max_len or max(lp.lens), lp.k_tq, lp.v_tq,
+                           1 / math.sqrt(lp.d), new_kv=new_kv, window=window, sinks=sinks, precise=precise, **src)
+
+
+@pytest.mark.parametrize("precise", [False, True])
+@pytest.mark.parametrize("d,B,hkv,G,lens,window,sinks", [
+    (128, 2, 2, 4, (300, 190), 100, 4),   # the window starts inside a page; sinks and tile padding
+    (256, 1, 1, 2, (2100,), 1000, 5),     # splits over the context
+    (64, 3, 2, 16, (70, 33, 1), 32, 4),   # flat rows, short sequences
+    (64, 1, 2, 4, (130,), None, 0),       # no window
+])
+def test_decode_step_at_both_precisions(cuda, d, B, hkv, G, lens, window, sinks, precise):
+    """Hidden positions take no weight in either form.  f16 operands: 2^-11
+    per operand, three of them in a row's weights and values (1e-3)."""
+    cache, g = _cache(cuda, d, 4, 4, B, hkv, lens, seed=d)
+    q = torch.randn(B, hkv * G, 1, d, generator=g)
+    got = _lib(cache, q.to(cuda), window, sinks, precise).cpu().numpy()[:, :, 0]
+    kd, vd = _decoded(cache, "k", B, hkv, d), _decoded(cache, "v", B, hkv, d)
+    want = np.zeros(got.shape)
+    for b, n in enumerate(lens):
+        pos = np.arange(n)
+        ok = np.ones(n, bool) if window is None else (pos >= n - window) | (pos < sinks)
+        for h in range(hkv * G):
+            want[b, h] = _attend(q[b, h].double().numpy(), kd[b, h // G, :n], vd[b, h // G, :n], 1 / math.sqrt(d), ok[None])[0]
+    err = _rel(got, want)
+    print(f"[lib decode d{d} lens {lens} w{window} precise {precise}] rel {err:.2e}", flush=True)
+    assert err < (1e-5 if precise else 1e-3)
