@@ -73,6 +73,7 @@ struct ChunkAttn {
   const float* signs;
   float oscale;                // V fragments' common scale, and of the un-rotation (direct output only)
   int64_t o_batch, o_row, o_head;  // output strides (elements) of a sequence, a query row and a head
+  int nan_zero;                // a row with a NaN score is zeros (decode steps); else NaN
 };
 
 // x of the lane 16 (32) lanes up or down: the butterfly pair of lane bit 4 (5)
@@ -411,12 +412,15 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
   for (int ct = 0; ct < CT; ++ct) {
     const float L = warp_sum_q(l_run[ct]);
     const float Z = ZM ? warp_sum_q(z_run[ct]) : 0.f;
-    const float inv = L > 0.f ? 1.f / L : 0.f;
+    // L == 0: no position.  A NaN score makes L NaN, which goes on to the output
+    // and, with splits, through the log-sum-exp to the merge.
+    const bool none = L == 0.f || (a.nan_zero != 0 && !(L > 0.f));
+    const float inv = none ? 0.f : 1.f / L;
     float y[NB][4];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[b][i] = L > 0.f ? (acc[ct][b][i] + Z) * inv : 0.f;
+      for (int i = 0; i < 4; ++i) y[b][i] = none ? 0.f : (acc[ct][b][i] + Z) * inv;
     const int col = wc0 + 16 * ct + n;
     const bool live = col < ncols;
     const int r = live ? col / a.G : 0, h = kvh * a.G + (live ? col - r * a.G : 0);
@@ -426,7 +430,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
 #pragma unroll
         for (int b = 0; b < NB; ++b)
           *reinterpret_cast<float4*>(a.wo + row * D + 16 * b + 4 * g) = make_float4(y[b][0], y[b][1], y[b][2], y[b][3]);
-        if (g == 0) a.wl[row] = L > 0.f ? m_run[ct] + __builtin_log2f(L) : -INFINITY;
+        if (g == 0) a.wl[row] = L == 0.f ? -INFINITY : m_run[ct] + __builtin_log2f(L);
       }
       continue;
     }

@@ -170,7 +170,8 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
     to[TK + tid] = ok ? 0.f : -INFINITY;
     to[3 * TK + tid] = 0.f;
     if (tnew[tid] < 0) {
-      to[tid] = ok ? dense[tid][0] * inv[0] : 0.f;
+      // an infinite norm stands for a NaN vector (its decode is infinity times the levels, rotated)
+      to[tid] = ok ? dense[tid][0] * inv[0] + (dense[tid][0] - dense[tid][0]) : 0.f;
       to[2 * TK + tid] = ok ? dense[tid][1] * inv[1] : 0.f;
     }
   }
@@ -189,12 +190,18 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
 #pragma unroll
       for (int i = 0; i < E; ++i) y[i] *= sign[l16 * E + i];
       fwht_lanes<E, 16>(y, l16);
-      float mx = 0.f;
+      float mx = 0.f, fin = 0.f;  // fin: NaN for a token with an infinity or a NaN
 #pragma unroll
       for (int i = 0; i < E; ++i) {
         y[i] *= 1.f / __builtin_sqrtf((float)D);
         mx = fmaxf(mx, fabsf(y[i]));
+        fin += y[i] * 0.f;
       }
+      fin += lane_xor<1>(fin);
+      fin += lane_xor<2>(fin);
+      fin += lane_xor<4>(fin);
+      fin += lane_xor<8>(fin);
+      const bool ok = fin == 0.f;
       mx = fmaxf(mx, lane_xor<1>(mx));
       mx = fmaxf(mx, lane_xor<2>(mx));
       mx = fmaxf(mx, lane_xor<4>(mx));
@@ -207,8 +214,12 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
       const int up = min(max(a - e + 127, 1), 253);
       const float f = __uint_as_float((uint32_t)up << 23);
 #pragma unroll
-      for (int i = 0; i < E; ++i) dense[t][l16 * E + i] = y[i] * f;
-      if (l16 == 0) to[(isv ? 2 * TK : 0) + t] = __uint_as_float((uint32_t)(254 - up) << 23) * (isv ? 256.f : 1.f);
+      for (int i = 0; i < E; ++i) dense[t][l16 * E + i] = ok ? y[i] * f : 0.f;
+      // a token that is not finite: operands of 0 and a NaN factor, so that the
+      // rows that attend it are NaN and the others (whose products meet its
+      // operands with a weight of 0) are not
+      if (l16 == 0)
+        to[(isv ? 2 * TK : 0) + t] = ok ? __uint_as_float((uint32_t)(254 - up) << 23) * (isv ? 256.f : 1.f) : __builtin_nanf("");
     }
   };
   if (any_new) {
@@ -339,7 +350,7 @@ __global__ __launch_bounds__(256) void chunk_merge_kernel(const float* __restric
                                                           int64_t rows, int hq_all, int hq_b, int splits,
                                                           const float* __restrict__ signs, float scale,
                                                           void* __restrict__ out, int64_t o_batch, int64_t o_row,
-                                                          int64_t o_head) {
+                                                          int64_t o_head, int nan_zero) {
   constexpr int E = D / 64;
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -347,12 +358,21 @@ __global__ __launch_bounds__(256) void chunk_merge_kernel(const float* __restric
   const float* lse = wl + r * splits;
   const float* po = wo + r * splits * D + lane * E;
   float M = -INFINITY;
-  for (int s = lane; s < splits; s += 64) M = fmaxf(M, lse[s]);
+  bool nan = false;  // a split with a NaN score; the maximum does not show it
+  for (int s = lane; s < splits; s += 64) {
+    M = fmaxf(M, lse[s]);
+    nan = nan || lse[s] != lse[s];
+  }
   M = wave_max64(M);
+  nan = __builtin_amdgcn_ballot_w64(nan) != 0;
   float y[E], W = 0.f;
 #pragma unroll
   for (int i = 0; i < E; ++i) y[i] = 0.f;
-  if (M != -INFINITY) {
+  if (nan) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) y[i] = nan_zero ? 0.f : __builtin_nanf("");
+    W = 1.f;
+  } else if (M != -INFINITY) {
     for (int s = 0; s < splits; ++s) {
       float x[E];
       load_f32_small<E>(po + (int64_t)s * D, x);
@@ -410,6 +430,7 @@ hipError_t lib_launch(const LibPlan& p, LibSource s, const void* q, int qt, int6
   a.wl = direct ? nullptr : reinterpret_cast<float*>(ws + p.o_l);
   a.out = out; a.ot = ot; a.rot = ROT_SIGNS; a.signs = s.vsign; a.oscale = osc;
   a.o_batch = o_batch; a.o_row = o_row; a.o_head = o_head;
+  a.nan_zero = decode;
   for (int i = 0; i < p.nseg; ++i) {
     a.seg0 = i * p.seg;
     a.seg1 = std::min(a.seg0 + p.seg, p.span);
@@ -427,9 +448,9 @@ hipError_t lib_launch(const LibPlan& p, LibSource s, const void* q, int qt, int6
   if (direct) return hipSuccess;
   const int64_t rows = (int64_t)nq * batch * hq;
   const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-  if (ot == F32) chunk_merge_kernel<D, F32><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head);
-  else if (ot == F16) chunk_merge_kernel<D, F16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head);
-  else chunk_merge_kernel<D, BF16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head);
+  if (ot == F32) chunk_merge_kernel<D, F32><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head, a.nan_zero);
+  else if (ot == F16) chunk_merge_kernel<D, F16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head, a.nan_zero);
+  else chunk_merge_kernel<D, BF16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head, a.nan_zero);
   return hipGetLastError();
 }
 

@@ -10,7 +10,8 @@
 //   ROT_MATRIX o <- o M^T, M = signs (row-major D x D fp32): un-rotation of v1 V
 //              rotated by a matrix strategy (x M)
 //   ROT_NONE   o unchanged
-// A row with every split empty (lse = -inf) is written as zeros.  With
+// A row with every split empty (lse = -inf) is written as zeros, one with a
+// split whose lse is NaN as NaN.  With
 // lse_out, the row's natural-log log-sum-exp of the scaled scores goes there
 // too (-inf for an empty row): ln 2 * (M + log2 sum_s w_s).
 //
@@ -129,8 +130,13 @@ __global__ __launch_bounds__(256) void merge_splits_kernel(const float* __restri
     }
   }
   float M = -INFINITY;
-  for (int s = lane; s < num_splits; s += 64) M = fmaxf(M, lse[s]);
+  bool nan = false;  // a NaN split; the maximum does not show it
+  for (int s = lane; s < num_splits; s += 64) {
+    M = fmaxf(M, lse[s]);
+    nan = nan || lse[s] != lse[s];
+  }
   M = wave_max64(M);
+  nan = __builtin_amdgcn_ballot_w64(nan) != 0;
   float y[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) y[i] = 0.f;
@@ -170,9 +176,10 @@ __global__ __launch_bounds__(256) void merge_splits_kernel(const float* __restri
       y[i] = (part[0][lane * E + i] + part[1][lane * E + i]) + (part[2][lane * E + i] + part[3][lane * E + i]);
   }
   if (!live) return;
+  if (nan) W = __builtin_nanf("");
   if (lse_out != nullptr && lane == 0)
-    lse_out[r] = (W > 0.f) ? (M + __builtin_log2f(W)) * 0.69314718055994531f : -INFINITY;
-  const float inv = (W > 0.f) ? 1.f / W : 0.f;
+    lse_out[r] = W == 0.f ? -INFINITY : (M + __builtin_log2f(W)) * 0.69314718055994531f;
+  const float inv = W == 0.f ? 0.f : 1.f / W;
 #pragma unroll
   for (int i = 0; i < E; ++i) y[i] *= inv;
   if constexpr (ROT == ROT_MATRIX) {

@@ -152,3 +152,16 @@ def test_chunk_workspace_rejects():
                 (16, 8, 2, 128, -1, 4, 4, 0, 0), (16, 8, 2, 128, 100, 5, 4, 0, 0), (16, 8, 2, 128, 100, 16, 4, 0, 0),
                 (16, 8, 2, 128, 2 ** 30, 4, 4, 0, 0)):
         assert f(*bad) == -1, bad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("past", [40, 3000])  # one split, several
+def test_a_nan_query_row_stays_nan(cuda, past):
+    layer, cache, row = _case(cuda, 64, 4, 4, 1, past + 20, True, 16, seed=6)
+    q = torch.randn(20, 4, 64, generator=torch.Generator().manual_seed(1)).to(cuda)
+    want = _chunk(layer, q, cache, row, past, 4, 4, True)
+    q[7, 2, 5] = float("nan")
+    got = _chunk(layer, q, cache, row, past, 4, 4, True)
+    assert torch.isnan(got[7, 2]).all()
+    got[7, 2] = want[7, 2]
+    assert _rel(got.cpu().numpy(), want.cpu().double().numpy()) < 1e-5

@@ -181,3 +181,39 @@ def test_decode_step_at_both_precisions(cuda, d, B, hkv, G, lens, window, sinks,
     err = _rel(got, want)
     print(f"[lib decode d{d} lens {lens} w{window} precise {precise}] rel {err:.2e}", flush=True)
     assert err < (1e-5 if precise else 1e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,past", [(64, 90), (64, 2100), (128, 90), (128, 2100)])  # one split, several
+def test_not_a_number_stays_in_its_rows(cuda, d, past, dtype):
+    """A NaN query row, an infinite new key and an infinite new value: the rows
+    that meet them are NaN (as softmax attention gives), the others as without."""
+    hkv, G, n = 2, 2, 24
+    cache, g = _cache(cuda, d, 4, 4, 1, hkv, (past,), seed=past, dtype=dtype)
+    k, v = (torch.randn(1, hkv, n, d, generator=g).to(dtype).to(cuda) for _ in range(2))
+    q = torch.randn(1, hkv * G, n, d, generator=g).to(dtype).to(cuda)
+    cache.store_compressed_kv(k, v, 0)
+    want = _lib(cache, q, new_kv=(k, v)).float().cpu()
+    q2, k2, v2 = q.clone(), k.clone(), v.clone()
+    q2[0, 1, 5, 3] = float("nan")        # kv head 0, row 5 of one head
+    k2[0, 0, 15, 7] = float("inf")       # kv head 0, rows 15 ..
+    v2[0, 1, 20, 9] = float("-inf")      # kv head 1, rows 20 ..
+    got = _lib(cache, q2, new_kv=(k2, v2)).float().cpu()
+    bad = torch.zeros(hkv * G, n, dtype=torch.bool)
+    bad[1, 5] = True
+    bad[:G, 15:] = True
+    bad[G:, 20:] = True
+    assert torch.isnan(got[0][bad]).all()
+    assert _rel(got[0][~bad].numpy(), want[0][~bad].numpy()) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("ctx", [90, 2100])  # one split, several
+def test_decode_step_with_an_infinite_key_norm(cuda, ctx):
+    """A row with a NaN score is zeros in a windowed decode step (softmax's NaN
+    weights count as 0), not an average of what the other splits hold."""
+    d, hkv, G = 64, 2, 2
+    cache, g = _cache(cuda, d, 4, 4, 1, hkv, (ctx,), seed=3)
+    cache._pages[0].kn[0, 0, ctx - 50] = float("inf")
+    q = torch.randn(1, hkv * G, d, generator=g).to(cuda)
+    got = cache.decode_attention(q, 0, 0.125, sliding_window=ctx - 10, sink_tokens=4).cpu()
+    assert (got[0, :G] == 0).all() and torch.isfinite(got).all() and (got[0, G:] != 0).any(dim=-1).all()
