@@ -46,6 +46,16 @@ __device__ __forceinline__ float table_pow2(const float* __restrict__ c, int n) 
   return __uint_as_float((uint32_t)min(max(263 - e, 1), 254) << 23);
 }
 
+// Common power of two of the weights' factors (the V scale's own power of two
+// is in the V operand, so that a factor is in [1, 2) times this; raw slots have
+// no scale): the largest with which 2^TAU = 16 times a factor stays an f16
+// number, so that the weights' low parts are normal numbers as far down as f16
+// has them.  With the tile-first sums of the attention kernel, one key that
+// takes most of the weight over 30000 others 24 log2 units below it, relative
+// error of raw d = 64 / K4 V4 d = 64 / K8 V8 d = 256 with factors of 1 / 32 /
+// 32 and one running sum: 1.8e-5 / 1.2e-5 / 1.3e-5; now 1.0e-6 / 8e-7 / 8e-7.
+__host__ __device__ constexpr float v_lift(bool raw, int vb) { return raw ? 2048.f : vb == 8 ? 512.f : 1024.f; }
+
 // One 32-token tile of one kv head: slots -> LDS rows -> fragments.
 template <int D, bool KHL>
 __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
@@ -124,7 +134,7 @@ __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
     }
     if (sub == 0) {
       const bool ok = tok_ok[t] != 0;
-      float fk = 1.f, vs = 1.f, vm = 0.f, ve = 1.f;
+      float fk = 1.f, vs = v_lift(true, vb), vm = 0.f, ve = 1.f;
       if (!raw) {
         if (!kf8) {
           const float kn = f16_bits_to_f32(row_bits(row, 8 * geo.mse, 16));
@@ -134,12 +144,11 @@ __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
         // V operand (code - mid) * 2^e, exact in f16, with the middle of the
         // code range moved into the minimum: the sums then have the outputs'
         // magnitude, not that of an offset the minimum cancels.  2^(e + 5) is the scale's own power
-        // of two, so that the weight's factor lies in [32, 64) and its low
-        // part stays a normal number for weights down to 2^-8; e held where
-        // the largest code stays finite and the codes normal
-        const int e = min(max((int)((sb >> 10) & 31u) - 20, -14), vb == 8 ? 8 : 12);
+        // of two, and e is held where the largest code stays finite and the
+        // codes normal
+        const int e = min(max((int)((sb >> 10) & 31u) - 20, -14), vb == 8 ? 9 : 12);
         ve = __uint_as_float((uint32_t)(127 + e) << 23);
-        vs = f16_bits_to_f32(sb) * __uint_as_float((uint32_t)(127 - e) << 23);
+        vs = f16_bits_to_f32(sb) * __uint_as_float((uint32_t)(127 - e) << 23) * (v_lift(false, vb) / 32.f);
         vm = __builtin_fmaf(mid, f16_bits_to_f32(sb), f16_bits_to_f32(row_bits(row, 8 * (geo.kps + geo.vdb) + 16, 16)));
       }
       float* o = tok + (int64_t)kvh * tstride + (int64_t)(tile * 32 / TK) * 4 * TK + (tile * 32) % TK + t;
@@ -283,6 +292,7 @@ hipError_t chunk_launch(const ChunkPlan& p, const void* q, int qt, int64_t q_row
   a.wo = direct ? nullptr : reinterpret_cast<float*>(ws + p.o_o);
   a.wl = direct ? nullptr : reinterpret_cast<float*>(ws + p.o_l);
   a.out = out; a.ot = ot; a.rot = vrot ? ROT_PLAIN : ROT_NONE; a.signs = nullptr;
+  a.vscale = raw ? 1.f / v_lift(true, vb) : 32.f / v_lift(false, vb);
   a.oscale = vrot ? fwht_scale(D) : 1.f;
   a.lens = nullptr; a.lens_less = 0; a.hkv_b = hkv;
   a.o_batch = 0; a.o_row = o_row; a.o_head = o_head;

@@ -71,7 +71,8 @@ struct ChunkAttn {
   void* out;                   // the output itself (wo == null)
   int ot, rot;                 // output dtype; MergeRot of the direct output (ROT_NONE / PLAIN / SIGNS)
   const float* signs;
-  float oscale;                // V fragments' common scale, and of the un-rotation (direct output only)
+  float vscale;                // of the accumulators: undoes the V operands' and factors' common power of two
+  float oscale;                // of the un-rotation (direct output only)
   int64_t o_batch, o_row, o_head;  // output strides (elements) of a sequence, a query row and a head
   int nan_zero;                // a row with a NaN score is zeros (decode steps); else NaN
 };
@@ -342,6 +343,10 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
       }
     }
     // what the high parts' products leave time for: the low parts and the sums
+    // (a tile's first, so that many small weights beside a large one count)
+    float lt[CT], zt[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) lt[ct] = zt[ct] = 0.f;
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
 #pragma unroll
@@ -351,8 +356,8 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
         for (int i = 0; i < 4; ++i) {
           const bool hid = edge && s[k][ct][i] < 0.f;
           const float e = hid ? 0.f : s[k][ct][i];
-          l_run[ct] += e;
-          if constexpr (ZM) z_run[ct] = __builtin_fmaf(e, hid ? 0.f : tf[k][3][i], z_run[ct]);
+          lt[ct] += e;
+          if constexpr (ZM) zt[ct] = __builtin_fmaf(e, hid ? 0.f : tf[k][3][i], zt[ct]);
           const half2_t hi = __builtin_bit_cast(half2_t, (uint32_t)ph[k >> 1][ct][2 * (k & 1) + (i >> 1)]);
           if constexpr (NH == 2) r[i] = __builtin_fmaf(e, hid ? 0.f : tf[k][2][i], -(float)hi[i & 1]);
         }
@@ -361,6 +366,11 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
           for (int h = 0; h < 2; ++h) pl[k >> 1][ct][2 * (k & 1) + h] = pk_f16(r[2 * h], r[2 * h + 1]);
         }
       }
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      l_run[ct] += lt[ct];
+      z_run[ct] += zt[ct];
     }
 #pragma unroll
     for (int part = VHL ? -1 : 0; part < NH; ++part)
@@ -420,7 +430,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[b][i] = none ? 0.f : (acc[ct][b][i] + Z) * inv;
+      for (int i = 0; i < 4; ++i) y[b][i] = none ? 0.f : __builtin_fmaf(acc[ct][b][i], a.vscale, Z) * inv;
     const int col = wc0 + 16 * ct + n;
     const bool live = col < ncols;
     const int r = live ? col / a.G : 0, h = kvh * a.G + (live ? col - r * a.G : 0);

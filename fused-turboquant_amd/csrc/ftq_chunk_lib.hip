@@ -45,6 +45,10 @@ struct LibSource {
   int window, sinks, vsinks;  // decode: window (0: none), sinks, and their virtual positions (a multiple of 32)
 };
 
+// Common power of two of the weights' factors: the largest with which 2^TAU =
+// 16 times the factor of the largest fp16 norm (2^16 / 2^7) stays below 2^16.
+constexpr float V_LIFT = 4.f;
+
 // bits [p, p + n) of a dword array with a pad dword, n <= 16
 __device__ __forceinline__ uint32_t word_bits(const uint32_t* w, int p, int n) {
   // both words always (no branch, so that the reads of several codes overlap)
@@ -155,12 +159,12 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
       tpos[t] = ok || nw >= 0 ? pos : -1;
       tnew[t] = nw;
       // V operand: level * 2^(ex + 8), near its norm; the weight's factor stays
-      // near [32, 64), so that small weights' low parts are normal f16 numbers
-      // (the 2^8 leaves with the output's scale)
+      // near [32, 64) V_LIFT, so that small weights' low parts are normal f16
+      // numbers (the 2^8 and V_LIFT leave with the accumulators' scale)
       const int ex = min(max((int)((vn >> 10) & 31u) - 20, -6), 7);
       vex[t] = __uint_as_float((uint32_t)(127 + 8 + ex) << 23);
       dense[t][0] = f16_bits_to_f32(kn);
-      dense[t][1] = f16_bits_to_f32(vn) * __uint_as_float((uint32_t)(127 - ex) << 23);
+      dense[t][1] = f16_bits_to_f32(vn) * __uint_as_float((uint32_t)(127 - ex) << 23) * V_LIFT;
     }
   }
   __syncthreads();
@@ -208,7 +212,7 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
       mx = fmaxf(mx, lane_xor<8>(mx));
       // K: largest magnitude to [512, 1024).  V: largest magnitude M to
       // [2^a, 2^(a+1)), a = log2 M + 3 within [2, 14]: the weight's factor
-      // M 2^(8 - a) is then in [32, 64) as for the codes
+      // M 2^(8 - a) is then in [32, 64) V_LIFT as for the codes
       const int e = (int)((__float_as_uint(mx) >> 23) & 255u) - 127;
       const int a = isv ? min(max(e + 3, 2), 14) : 9;
       const int up = min(max(a - e + 127, 1), 253);
@@ -219,7 +223,7 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
       // rows that attend it are NaN and the others (whose products meet its
       // operands with a weight of 0) are not
       if (l16 == 0)
-        to[(isv ? 2 * TK : 0) + t] = ok ? __uint_as_float((uint32_t)(254 - up) << 23) * (isv ? 256.f : 1.f) : __builtin_nanf("");
+        to[(isv ? 2 * TK : 0) + t] = ok ? __uint_as_float((uint32_t)(254 - up) << 23) * (isv ? 256.f * V_LIFT : 1.f) : __builtin_nanf("");
     }
   };
   if (any_new) {
@@ -424,11 +428,11 @@ hipError_t lib_launch(const LibPlan& p, LibSource s, const void* q, int qt, int6
     a.lens = s.lens; a.lens_less = nq; a.past = max_len - nq; a.window = decode ? 0 : s.window;
   }
   if (!decode) s.window = 0;  // virtual positions are a decode step's
-  const float osc = rs * (1.f / 256.f);  // V operands carry 2^8
+  a.vscale = 1.f / (256.f * V_LIFT);
   const bool direct = a.splits_all == 1;
   a.wo = direct ? nullptr : reinterpret_cast<float*>(ws + p.o_o);
   a.wl = direct ? nullptr : reinterpret_cast<float*>(ws + p.o_l);
-  a.out = out; a.ot = ot; a.rot = ROT_SIGNS; a.signs = s.vsign; a.oscale = osc;
+  a.out = out; a.ot = ot; a.rot = ROT_SIGNS; a.signs = s.vsign; a.oscale = rs;
   a.o_batch = o_batch; a.o_row = o_row; a.o_head = o_head;
   a.nan_zero = decode;
   for (int i = 0; i < p.nseg; ++i) {
@@ -448,9 +452,9 @@ hipError_t lib_launch(const LibPlan& p, LibSource s, const void* q, int qt, int6
   if (direct) return hipSuccess;
   const int64_t rows = (int64_t)nq * batch * hq;
   const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-  if (ot == F32) chunk_merge_kernel<D, F32><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head, a.nan_zero);
-  else if (ot == F16) chunk_merge_kernel<D, F16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head, a.nan_zero);
-  else chunk_merge_kernel<D, BF16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, osc, out, o_batch, o_row, o_head, a.nan_zero);
+  if (ot == F32) chunk_merge_kernel<D, F32><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, rs, out, o_batch, o_row, o_head, a.nan_zero);
+  else if (ot == F16) chunk_merge_kernel<D, F16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, rs, out, o_batch, o_row, o_head, a.nan_zero);
+  else chunk_merge_kernel<D, BF16><<<grid, block, 0, st>>>(a.wo, a.wl, rows, batch * hq, hq, a.splits_all, s.vsign, rs, out, o_batch, o_row, o_head, a.nan_zero);
   return hipGetLastError();
 }
 

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256, 2) void v1_attn_split_kernel(
   }
   const float qf = qinv[(!QL && m >= 8) ? m - 8 : m] * tsc_inv;  // of the lane's column (head)
 
-  constexpr float TAU = 4.f, MINF = -3.0e38f, MID = 0.5f * (float)((1 << VB) - 1);
+  constexpr float V_LIFT = 32.f, TAU = 4.f, MINF = -3.0e38f, MID = 0.5f * (float)((1 << VB) - 1);
   float m_run = MINF, l_run = 0.f, z_run = 0.f;
   floatx4 acc[NB];
 #pragma unroll
@@ -310,11 +310,12 @@ __global__ __launch_bounds__(256, 2) void v1_attn_split_kernel(
       const float sc = (float)__builtin_bit_cast(_Float16, (uint16_t)cur.vs[st]);
       const float mn = (float)__builtin_bit_cast(_Float16, (uint16_t)cur.vm[st]);
       // V operand (code - mid) 2^e: 2^(e + 5) the scale's own power of two (its
-      // factor in [32, 64), so that small weights' low parts stay normal), e
-      // where codes stay normal and (2^VB + mid) 2^e finite
+      // factor in [32, 64) V_LIFT, so that small weights' low parts stay normal:
+      // 16 times it is the largest f16), e where codes stay normal and (2^VB +
+      // mid) 2^e finite
       const int e = min(max((int)((cur.vs[st] >> 10) & 31u) - 20, -14), 11);
       const float x = g == 0 ? kn / __builtin_sqrtf(csq + 1e-16f)
-                    : g == 1 ? sc * __uint_as_float((uint32_t)(127 - e) << 23)
+                    : g == 1 ? sc * (V_LIFT * __uint_as_float((uint32_t)(127 - e) << 23))
                     : g == 2 ? __builtin_fmaf(MID, sc, mn)
                              : __uint_as_float((uint32_t)(127 + e) << 23);
       fields[wave][st][g][m] = x;
@@ -369,14 +370,15 @@ __global__ __launch_bounds__(256, 2) void v1_attn_split_kernel(
     Op8 pb, pl;
     half2_t e2[4], c2[4];  // 2^(e + VB) and -(2^VB + mid) 2^e of the operand pairs' tokens
     const bool lo_col = !QL && m >= 8;
+    float lt = 0.f, zt = 0.f;  // the tile's sums first: many small weights beside a large one count
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
       float w[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float p = __builtin_amdgcn_exp2f(s[st][i] - m_run);
-        l_run += p;
-        z_run = __builtin_fmaf(p, vz[st][i], z_run);
+        lt += p;
+        zt = __builtin_fmaf(p, vz[st][i], zt);
         w[i] = p * vf[st][i];
       }
 #pragma unroll
@@ -391,6 +393,8 @@ __global__ __launch_bounds__(256, 2) void v1_attn_split_kernel(
         c2[2 * st + h] = ex * (_Float16)(-((float)(1 << VB) + MID));
       }
     }
+    l_run += lt;
+    z_run += zt;
     constexpr uint32_t CM = ((1u << VB) - 1u) << (10 - VB);
 #pragma unroll
     for (int ch = 0; ch < Q::NCH; ++ch) {
@@ -454,7 +458,7 @@ __global__ __launch_bounds__(256, 2) void v1_attn_split_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       // row 4g + i of accumulator bb is dim NB (4g + i) + bb
-      const float o = QL ? acc[bb][i] : acc[bb][i] + dpp_xor8(acc[bb][i]);
+      const float o = (QL ? acc[bb][i] : acc[bb][i] + dpp_xor8(acc[bb][i])) * (1.f / V_LIFT);
       if (m < G) red_o[(wave * G + m) * (D + 1) + NB * (4 * g + i) + bb] = o;
     }
   __syncthreads();

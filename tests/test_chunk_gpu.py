@@ -165,3 +165,30 @@ def test_a_nan_query_row_stays_nan(cuda, past):
     assert torch.isnan(got[7, 2]).all()
     got[7, 2] = want[7, 2]
     assert _rel(got.cpu().numpy(), want.cpu().double().numpy()) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("below", [20, 24])
+@pytest.mark.parametrize("d,bits", [(64, RAW), (128, RAW), (256, RAW), (64, 4), (256, 8)])
+def test_one_dominant_key_and_a_long_tail(cuda, d, bits, below):
+    """One key takes most of the weight; 30000 others, ``below`` log2 units
+    under it, together still move the output."""
+    from fused_turboquant import raw as R, v1 as V1
+    n, past, G = 16, 30000, 2
+    L, nb = past + n, (past + n + 15) // 16
+    g = torch.Generator().manual_seed(d)
+    k, v = torch.randn(L, 1, d, generator=g) * 0.02, torch.randn(L, 1, d, generator=g) * 0.5 + 0.5
+    u = torch.randn(d, generator=g)
+    u /= u.norm()
+    k[0, 0] = 30 * u
+    q = torch.randn(n, G, d, generator=g) * 0.05 + u * (below * math.log(2) * math.sqrt(d) / 30)
+    row, slots = torch.arange(nb, dtype=torch.int32, device=cuda), torch.arange(L, device=cuda)
+    layer = None if bits == RAW else V1.TurboQuantV1Layer(d, bits, bits, device=cuda)
+    shape = (nb, 16, 1, 4 * d) if layer is None else layer.kv_cache_shape(nb, 16, 1)
+    cache = torch.zeros(shape, dtype=torch.uint8, device=cuda)
+    (R.raw_store if layer is None else layer.store)(k.to(cuda), v.to(cuda), cache, slots)
+    got = _chunk(layer, q.to(cuda), cache, row, past, bits, bits, False).cpu().numpy()
+    want = _want(layer, q, cache, row, past, bits, bits, False)
+    err = _rel(got, want)
+    print(f"[chunk tail d{d} bits {bits} below {below}] rel {err:.2e}", flush=True)
+    assert err < 1e-5
