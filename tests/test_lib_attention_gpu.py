@@ -3,10 +3,11 @@ HuggingFace cache): windowed and flat decode steps and multi-token steps,
 against float64 attention over the oracle's decode of the stored codes (and,
 for a multi-token step, the new tokens as given).
 
-Tolerances (relative 2-norm on fp32 outputs): decode steps and float32
-multi-token steps carry f16 hi + lo operands (2^-22) with fp32 sums: 1e-5.
-16-bit multi-token steps carry f16 operands, each with a relative error of at
-most 2^-11 (1e-3 on the outputs, whose own rounding is 2^-9 for bf16).
+Tolerances (relative 2-norm): decode steps and float32 and float16 multi-token
+steps carry f16 hi + lo operands (2^-22) with fp32 sums: 1e-5, and for float16
+outputs their own rounding, at most 2^-11.  bfloat16 multi-token steps carry
+f16 operands, each with a relative error of at most 2^-11 (1e-3 on the outputs,
+whose own rounding is 2^-9).
 """
 import math
 
@@ -108,7 +109,7 @@ def test_multi_token_step(cuda, d, bk, bv, B, hkv, G, past, n, window, dtype):
             want[b, h] = _attend(q[b, h].double().numpy(), kk, vv, 1 / math.sqrt(d), ok)
     err = _rel(got.float().cpu().numpy(), want)
     print(f"[lib chunk d{d} K{bk}V{bv} past {past} n {n} w{window} {dtype}] rel {err:.2e}", flush=True)
-    assert err < {torch.float32: 1e-5, torch.float16: 1e-3 + 2.0 ** -11, torch.bfloat16: 1e-3 + 2.0 ** -9}[dtype]
+    assert err < {torch.float32: 1e-5, torch.float16: 1e-5 + 2.0 ** -11, torch.bfloat16: 1e-3 + 2.0 ** -9}[dtype]
 
 
 def test_large_values_stay_finite(cuda):
@@ -217,3 +218,22 @@ def test_decode_step_with_an_infinite_key_norm(cuda, ctx):
     q = torch.randn(1, hkv * G, d, generator=g).to(cuda)
     got = cache.decode_attention(q, 0, 0.125, sliding_window=ctx - 10, sink_tokens=4).cpu()
     assert (got[0, :G] == 0).all() and torch.isfinite(got).all() and (got[0, G:] != 0).any(dim=-1).all()
+
+
+@pytest.mark.parametrize("d,past,n", [(64, 49, 300), (128, 27, 120), (256, 82, 31)])
+def test_float16_step_keeps_its_operands(cuda, d, past, n):
+    """float16 queries and new tokens are not rounded on their way to the
+    products: with scores of up to 2^5, f16 operands would show (7e-4 to 8e-4)."""
+    hkv, G, dt = 1, 4, torch.float16
+    cache, g = _cache(cuda, d, 4, 4, 1, hkv, (past,), seed=d, dtype=dt)
+    kd, vd = (np.ascontiguousarray(_decoded(cache, w, 1, hkv, d)[:, :, :past]) for w in "kv")
+    k, v = (torch.randn(1, hkv, n, d, generator=g).to(dt) for _ in range(2))
+    q = (6 * torch.randn(1, hkv * G, n, d, generator=g)).to(dt)
+    cache.store_compressed_kv(k.to(cuda), v.to(cuda), 0)
+    got = cache.chunk_attention(q.to(cuda), k.to(cuda), v.to(cuda), 0, 1 / math.sqrt(d)).float().cpu().numpy()[0]
+    kk, vv = (np.concatenate([x[0, 0], y[0, 0].double().numpy()]) for x, y in ((kd, k), (vd, v)))
+    ok = np.arange(past + n)[None] <= past + np.arange(n)[:, None]
+    want = np.stack([_attend(q[0, h].double().numpy(), kk, vv, 1 / math.sqrt(d), ok) for h in range(G)])
+    err = _rel(got, want)
+    print(f"[lib chunk float16 d{d} past {past} n {n}] rel {err:.2e}", flush=True)
+    assert err < 1e-5 + 2.0 ** -11  # the products, and one rounding of the output
