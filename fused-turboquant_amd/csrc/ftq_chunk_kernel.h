@@ -58,7 +58,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct ChunkAttn {
   const u32x4 *kf, *vf, *qf;   // fragments: [kv head][...]
   const float* tok;            // [kv head][tile][4][TK]: K factor, bias, V factor, V minimum
-  const float* qfac;           // per column factor of the scores ([kv head][column]); KHL only
+  const float* qfac;           // per column factor of the scores ([kv head][column]); KHL and NH == 1
   int64_t kstride, vstride, qstride;  // uint4 per kv head
   int64_t tstride;             // floats per kv head
   int cstride;                 // columns per kv head (qfac)
@@ -178,6 +178,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
   // the query operands of the wave's columns
   half8 qh[CT][NS], ql[NH == 2 ? CT : 1][NH == 2 ? NS : 1];
   float qs[CT];
+  bool qlarge = false;  // NH == 1: a column whose query was scaled to stay an f16 number; rare
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const u32x4* pq = a.qf + (int64_t)kvh * a.qstride + (int64_t)(wc0 / 16 + ct) * (NS * NH * 64) + lane;
@@ -186,7 +187,9 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
       qh[ct][s] = __builtin_bit_cast(half8, pq[(s * NH) * 64]);
       if constexpr (NH == 2) ql[ct][s] = __builtin_bit_cast(half8, pq[(s * NH + 1) * 64]);
     }
-    qs[ct] = KHL ? a.qfac[(int64_t)kvh * a.cstride + wc0 + 16 * ct + n] : 1.f;
+    qs[ct] = KHL || NH == 1 ? a.qfac[(int64_t)kvh * a.cstride + wc0 + 16 * ct + n] : 1.f;
+    if constexpr (!KHL && NH == 1)
+      qlarge = qlarge || __builtin_amdgcn_ballot_w64(qs[ct] > 1.f && wc0 + 16 * ct + n < ncols) != 0;  // wave-uniform
   }
 
   constexpr float TAU = 4.f;        // weights stay below 2^TAU
@@ -284,6 +287,14 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
     // each of them.
     __builtin_amdgcn_sched_barrier(0);
     if (more) fetch(t + 1, p ^ 1);
+    if constexpr (!KHL && NH == 1) {
+      if (qlarge) {
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) s[k][ct] *= qs[ct];
+      }
+    }
     // scores: x K factor (and the column's), + bias; masked on the edges
 #pragma unroll
     for (int k = 0; k < NT; ++k)
@@ -487,7 +498,8 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void chunk_attn_kernel(const
 // (H, or x M), times qscale, to fragments of NH f16 parts.  KHL: each query is
 // first scaled by the power of two that puts its largest magnitude in
 // [256, 512), so that the low parts of the others stay normal f16 numbers;
-// qfac takes the inverse.
+// qfac takes the inverse.  NH == 1: only a query that f16 cannot hold is scaled,
+// to [2^13, 2^14), and qfac is 1 for the others.
 template <int D, int QT, int NH, bool KHL>
 __global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict__ query, int64_t q_batch,
                                                           int64_t q_row, int64_t q_head, int nq, int hq, int hkv, int hq_b, const float* __restrict__ signs,
@@ -511,7 +523,7 @@ __global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict
   if (rot != nullptr) rot_matrix_lanes<D, E>(y, rot, rows[grp], l16);
   else if (rotate) fwht_lanes<E, 16>(y, l16);
   float up = 1.f;
-  if constexpr (KHL) {
+  if constexpr (KHL || NH == 1) {
     float mx = 0.f;
 #pragma unroll
     for (int i = 0; i < E; ++i) {
@@ -523,7 +535,8 @@ __global__ __launch_bounds__(256) void chunk_query_kernel(const void* __restrict
     mx = fmaxf(mx, lane_xor<4>(mx));
     mx = fmaxf(mx, lane_xor<8>(mx));
     const int e = (int)((__float_as_uint(mx) >> 23) & 255u);  // mx in [2^(e-127), 2^(e-126))
-    const int ue = min(max(135 + 127 - e, 1), 253);           // 2^(8 - (e - 127)), kept normal both ways
+    int ue = min(max(135 + 127 - e, 1), 253);                 // 2^(8 - (e - 127)), kept normal both ways
+    if constexpr (!KHL) ue = e >= 127 + 14 && e < 255 ? 140 + 127 - e : 127;
     up = __uint_as_float((uint32_t)ue << 23);
     if (live && l16 == 0) qfac[(int64_t)kvh * cstride + col] = __uint_as_float((uint32_t)(254 - ue) << 23);
   } else {

@@ -342,7 +342,7 @@ bool lib_plan(LibPlan& p, int batch, int nq, int hq, int hkv, int d, int max_len
   p.o_v = take(p.vstride * units * 16);
   p.o_t = take(p.tstride * units * 4);
   p.o_q = take(p.qstride * units * 16);
-  p.o_f = take(prec ? p.colpad * units * 4 : 0);
+  p.o_f = take(p.colpad * units * 4);
   const int64_t all = (int64_t)p.nseg * p.splits, rows = (int64_t)nq * hq * batch * all;
   p.o_o = take(all > 1 ? rows * d * 4 : 0);
   p.o_l = take(all > 1 ? rows * 4 : 0);

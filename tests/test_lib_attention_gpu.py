@@ -237,3 +237,24 @@ def test_float16_step_keeps_its_operands(cuda, d, past, n):
     err = _rel(got, want)
     print(f"[lib chunk float16 d{d} past {past} n {n}] rel {err:.2e}", flush=True)
     assert err < 1e-5 + 2.0 ** -11  # the products, and one rounding of the output
+
+
+def test_queries_beyond_f16(cuda):
+    """bfloat16 queries larger than f16 holds, with keys so small that their
+    scores are ordinary, beside ordinary rows."""
+    d, hkv, G, past, n, dt = 128, 2, 2, 40, 20, torch.bfloat16
+    cache, g = _cache(cuda, d, 4, 4, 1, hkv, (past,), seed=2, dtype=dt)
+    k, v = (torch.randn(1, hkv, n, d, generator=g) for _ in range(2))
+    q = torch.randn(1, hkv * G, n, d, generator=g)
+    k, v, q = k.to(dt), v.to(dt), q.to(dt)
+    cache.store_compressed_kv(k.to(cuda), v.to(cuda), 0)
+    big = q.clone()
+    big[:, 1, 3:] *= 2.0 ** 20  # powers of two: exact, so that the key's factor brings the same scores back
+    cache._pages[0].kv_cache.zero_()  # the past's norms are 0: its scores are 0 for every query
+    want = _lib(cache, q.to(cuda), new_kv=(k.to(cuda), v.to(cuda))).float().cpu()
+    k2 = k.clone()
+    k2[:, 0] *= 2.0 ** -20
+    got = _lib(cache, big.to(cuda), new_kv=(k2.to(cuda), v.to(cuda))).float().cpu()
+    assert torch.isfinite(got).all()
+    assert _rel(got[0, 1, 3:].numpy(), want[0, 1, 3:].numpy()) < 1e-3 + 2.0 ** -8
+    assert _rel(got[0, G:].numpy(), want[0, G:].numpy()) < 1e-6
