@@ -77,6 +77,7 @@ __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
   const float mid = raw ? 0.f : 0.5f * (float)((1 << vb) - 1);
   const int pos0 = seg0 + tile * 32;
 
+  float beyond = 0.f;  // raw slots: whether this lane read a V element that is not finite
   {  // 8 lanes a token, 16 bytes (or 4 dwords) each
     const int t = tid >> 3, sub = tid & 7;
     const int pos = pos0 + t, page = pos >> lbs;
@@ -99,6 +100,11 @@ __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (4 * c + j < nd) dst[4 * c + j] = w[j];
+      if (raw && c >= D / 8) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if ((w[j] & 0x7c00u) == 0x7c00u || (w[j] & 0x7c000000u) == 0x7c000000u) beyond = 1.f;
+      }
     }
     if (sub == 0) tok_ok[t] = ok;
   }
@@ -132,9 +138,13 @@ __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
       }
       csq = group_sum<8>(csq);
     }
+    if (raw) beyond = group_sum<8>(beyond);
     if (sub == 0) {
       const bool ok = tok_ok[t] != 0;
-      float fk = 1.f, vs = v_lift(true, vb), vm = 0.f, ve = 1.f;
+      // A raw V that is not finite (a bf16 value beyond fp16's range): operands of
+      // 0 and a NaN factor, so that the rows that attend it are NaN and those
+      // whose products only meet it with a weight of 0 are not.
+      float fk = 1.f, vs = beyond == 0.f ? v_lift(true, vb) : __builtin_nanf(""), vm = 0.f, ve = beyond == 0.f ? 1.f : 0.f;
       if (!raw) {
         if (!kf8) {
           const float kn = f16_bits_to_f32(row_bits(row, 8 * geo.mse, 16));
@@ -194,7 +204,8 @@ __global__ __launch_bounds__(256) void chunk_gather_v1_kernel(
     for (int j = 0; j < 4; ++j) {
       const int t = (j >> 1) * 16 + 4 * g + 2 * (j & 1);
       if (raw) {
-        w[j] = row_bits(rows + t * pitch, 16 * D + 16 * d, 16) | (row_bits(rows + (t + 1) * pitch, 16 * D + 16 * d, 16) << 16);
+        w[j] = (vex[t] != 0.f ? row_bits(rows + t * pitch, 16 * D + 16 * d, 16) : 0u) |
+               (vex[t + 1] != 0.f ? row_bits(rows + (t + 1) * pitch, 16 * D + 16 * d, 16) << 16 : 0u);
       } else {
         const float x = ((float)row_bits(rows + t * pitch, 8 * geo.kps + d * vb, vb) - mid) * vex[t];
         const float y = ((float)row_bits(rows + (t + 1) * pitch, 8 * geo.kps + d * vb, vb) - mid) * vex[t + 1];

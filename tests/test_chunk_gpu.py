@@ -192,3 +192,17 @@ def test_one_dominant_key_and_a_long_tail(cuda, d, bits, below):
     err = _rel(got, want)
     print(f"[chunk tail d{d} bits {bits} below {below}] rel {err:.2e}", flush=True)
     assert err < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,past", [(64, 40), (128, 40), (256, 3000)])
+def test_an_infinite_raw_value_stays_in_the_rows_that_attend_it(cuda, d, past):
+    n, G, at = 30, 2, 12  # the 13th new token; 12 rows of its tile come before it
+    _, cache, row = _case(cuda, d, RAW, RAW, 1, past + n, False, 16, seed=7)
+    q = torch.randn(n, G, d, generator=torch.Generator().manual_seed(1)).to(cuda)
+    want = _chunk(None, q, cache, row, past, RAW, RAW, False)
+    v = cache[row[(past + at) // 16].long(), (past + at) % 16, 0].view(torch.float16)
+    v[d + 5], v[2 * d - 1] = float("inf"), float("nan")
+    got = _chunk(None, q, cache, row, past, RAW, RAW, False)
+    assert torch.equal(got[:at], want[:at])
+    assert torch.isnan(got[at:, :, [5, d - 1]]).all()
