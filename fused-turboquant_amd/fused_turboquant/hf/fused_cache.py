@@ -306,7 +306,7 @@ class CompressedKVCache(DynamicCache):
         if isinstance(lp, _LayerPages) and sliding_window is None:
             return P.paged_decode_attention(query, lp.kv_cache, lp.block_table, lp.lens_dev, lp.k_tq, lp.v_tq,
                                             scale=scale, max_seq_len=max(lp.lens))
-        if self._fused_attention(lp, query):
+        if self._fused_attention(lp, query, sliding_window):
             return self._lib_attention(lp, query.unsqueeze(2), scale, window=sliding_window,
                                        sinks=sink_tokens).squeeze(2)
         kd = self.decode_keys(layer_idx)
@@ -327,10 +327,12 @@ class CompressedKVCache(DynamicCache):
         return torch.matmul(w, _repeat_kv(vd, n_rep)).squeeze(2).to(query.dtype)
 
     @staticmethod
-    def _fused_attention(lp, query: torch.Tensor) -> bool:
-        """Whether the library-format attention kernels take this layer and query."""
+    def _fused_attention(lp, query: torch.Tensor, window: Optional[int] = None) -> bool:
+        """Whether the library-format attention kernels take this layer, query and
+        window (one that holds no position, and one sequence read by several
+        queries, stay with torch)."""
         hq, d = query.shape[1], query.shape[-1]
-        return (not _needs_grad(query) and d == lp.d and d in P.LIB_ATTENTION_DIMS and hq % lp.hkv == 0 and hq // lp.hkv <= 16
+        return (not _needs_grad(query) and query.shape[0] == lp.B and (window is None or window > 0) and d == lp.d and d in P.LIB_ATTENTION_DIMS and hq % lp.hkv == 0 and hq // lp.hkv <= 16
                 and lp.B * lp.hkv <= 65535 and query.dtype in (torch.float32, torch.float16, torch.bfloat16))
 
     @staticmethod
@@ -347,7 +349,7 @@ class CompressedKVCache(DynamicCache):
         compressed past and the step's own tokens, causal.  None where the
         kernels do not take the layer."""
         lp = self._pages[layer_idx]
-        if not self._fused_attention(lp, query) or _needs_grad(key, value) or key.dtype != value.dtype \
+        if not self._fused_attention(lp, query, sliding_window) or _needs_grad(key, value) or key.dtype != value.dtype \
                 or key.dtype not in (torch.float32, torch.float16, torch.bfloat16):
             return None
         return self._lib_attention(lp, query, scale, new_kv=(key, value), window=sliding_window)

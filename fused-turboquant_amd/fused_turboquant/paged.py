@@ -221,13 +221,17 @@ def lib_attention(query: torch.Tensor, lens: torch.Tensor, max_len: int, k_quant
     nk = nv = None
     if new_kv is not None:
         nk, nv = _rows16(new_kv[0]), _rows16(new_kv[1])
+    # beyond the context a window hides nothing and a sink is no position
+    most = max(int(max_len), 1)
+    window = min(int(window), most) if window else 0
+    sinks = min(max(int(sinks), 0), most) if window else 0
     kq, vq = k_quant.quantizer, v_quant.quantizer
     codes_k, codes_v, norms_k, norms_v, bt = ((pages[0], None, None, None, pages[1]) if pages is not None else
                                               (flat[0], flat[2], flat[1], flat[3], None))
     _lib.require_device(q, codes_k, lens, out)
     _ops.ops().lib_attention(q, codes_k, codes_v, norms_k, norms_v, bt, lens, nk, nv, k_quant.rotation.signs,
                              v_quant.rotation.signs, kq.levels, vq.levels, k_quant.bits, v_quant.bits, int(max_len),
-                             float(scale), int(window or 0), int(sinks) if window else 0, bool(precise), out)
+                             float(scale), window, sinks, bool(precise), out)
     return out
 
 

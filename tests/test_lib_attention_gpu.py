@@ -258,3 +258,19 @@ def test_queries_beyond_f16(cuda):
     assert torch.isfinite(got).all()
     assert _rel(got[0, 1, 3:].numpy(), want[0, 1, 3:].numpy()) < 1e-3 + 2.0 ** -8
     assert _rel(got[0, G:].numpy(), want[0, G:].numpy()) < 1e-6
+
+
+@pytest.mark.parametrize("window,sinks,queries", [
+    (0, 4, 1), (0, 0, 1), (-3, 2, 1),            # a window that holds no position
+    (2 ** 40, 4, 1), (20, -1, 1), (20, 2 ** 40, 1),  # beyond the context, no sinks, all of them
+    (20, 4, 3),                                  # one sequence read by three queries
+])
+@pytest.mark.parametrize("d", [64, 128])
+def test_windows_sinks_and_batches_of_the_torch_form(cuda, d, window, sinks, queries, monkeypatch):
+    """What the cache's torch form takes, the kernels or that form still take."""
+    cache, g = _cache(cuda, d, 4, 4, 1, 2, (50,), seed=4)
+    q = torch.randn(queries, 4, d, generator=g).to(cuda)
+    got = cache.decode_attention(q, 0, 0.1, sliding_window=window, sink_tokens=sinks).cpu()
+    monkeypatch.setattr(type(cache), "_fused_attention", staticmethod(lambda *a: False))
+    want = cache.decode_attention(q, 0, 0.1, sliding_window=window, sink_tokens=sinks).cpu()
+    assert got.shape == want.shape and (got - want).norm() <= 1e-5 * want.norm()
