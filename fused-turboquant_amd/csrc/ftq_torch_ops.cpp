@@ -50,6 +50,14 @@ void contig(const at::Tensor& t, const char* name) {
   TORCH_CHECK(t.is_contiguous(), "fused_tq: ", name, " must be contiguous");
 }
 
+// t with rows that kernels can read in 16-byte steps: itself, or an aligned copy
+// (contiguous() returns a contiguous view at any storage offset as it is)
+at::Tensor rows16(const at::Tensor& t) {
+  bool ok = t.dim() > 0 && t.stride(-1) == 1 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+  for (int64_t i = 0; ok && i + 1 < t.dim(); ++i) ok = t.stride(i) % 8 == 0;
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 void* stream_of(const at::Tensor& t) {
   return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
@@ -280,19 +288,21 @@ void v1_chunk_attention(const at::Tensor& query, const at::Tensor& kv_cache, con
 
 // ---- library-format attention: windows, other head dims, several tokens ----
 
-void lib_attention(const at::Tensor& query, const at::Tensor& codes_k, const std::optional<at::Tensor>& codes_v,
+void lib_attention(const at::Tensor& query_in, const at::Tensor& codes_k, const std::optional<at::Tensor>& codes_v,
                    const std::optional<at::Tensor>& norms_k, const std::optional<at::Tensor>& norms_v,
                    const std::optional<at::Tensor>& block_table, const at::Tensor& lens,
-                   const std::optional<at::Tensor>& new_key, const std::optional<at::Tensor>& new_value,
+                   std::optional<at::Tensor> new_key, std::optional<at::Tensor> new_value,
                    const at::Tensor& k_signs, const at::Tensor& v_signs, const at::Tensor& k_levels,
                    const at::Tensor& v_levels, int64_t bits_k, int64_t bits_v, int64_t max_len, double scale,
                    int64_t window, int64_t sinks, bool precise, at::Tensor& out) {
-  on_device(query, "query");
+  on_device(query_in, "query");
   on_device(out, "out");
   contig(codes_k, "codes_k");
   contig(lens, "lens");
-  TORCH_CHECK(query.dim() == 4 && out.sizes() == query.sizes() && query.stride(3) == 1 && out.stride(3) == 1,
-              "fused_tq: query and out must be [B, Hq, n, d] with contiguous rows");
+  TORCH_CHECK(query_in.dim() == 4 && out.sizes() == query_in.sizes() && out.stride(3) == 1,
+              "fused_tq: query and out must be [B, Hq, n, d], out with contiguous rows");
+  const c10::DeviceGuard g(query_in.device());
+  const at::Tensor query = rows16(query_in);
   TORCH_CHECK(lens.scalar_type() == at::kInt && lens.numel() == query.size(0), "fused_tq: lens must be int32 [B]");
   TORCH_CHECK(codes_k.scalar_type() == at::kByte && codes_k.dim() == 4, "fused_tq: codes_k must be uint8, 4-D");
   TORCH_CHECK_VALUE(max_len >= 0 && max_len <= INT32_MAX && window >= 0 && window <= INT32_MAX && sinks >= 0 &&
@@ -352,17 +362,17 @@ void lib_attention(const at::Tensor& query, const at::Tensor& codes_k, const std
   if (new_key.has_value()) {
     TORCH_CHECK(new_value.has_value() && new_key->dim() == 4 && new_key->sizes() == new_value->sizes() &&
                     new_key->size(0) == B && new_key->size(1) == hkv && new_key->size(2) == query.size(2) &&
-                    new_key->size(3) == d && new_key->stride(3) == 1 && new_value->stride(3) == 1 &&
-                    new_key->scalar_type() == new_value->scalar_type(),
-                "fused_tq: new keys and values must be [B, Hkv, n, d] with contiguous rows");
+                    new_key->size(3) == d && new_key->scalar_type() == new_value->scalar_type(),
+                "fused_tq: new keys and values must be [B, Hkv, n, d] of one type");
     on_device(*new_key, "new_key");
     on_device(*new_value, "new_value");
+    new_key = rows16(*new_key);
+    new_value = rows16(*new_value);
     a.new_key = new_key->data_ptr(); a.new_value = new_value->data_ptr(); a.new_dtype = dt(*new_key);
     a.k_batch = new_key->stride(0); a.k_head = new_key->stride(1); a.k_tok = new_key->stride(2);
     a.v_batch = new_value->stride(0); a.v_head = new_value->stride(1); a.v_tok = new_value->stride(2);
   }
   a.scale = (float)scale; a.window = (int)window; a.sinks = (int)sinks; a.precise = precise ? 1 : 0;
-  const c10::DeviceGuard g(query.device());
   if (B == 0 || query.size(2) == 0) return;
   const int64_t need = ftq_lib_attention_workspace_bytes(a.batch, a.n_query, a.num_q_heads, a.num_kv_heads, a.d,
                                                          a.max_len, a.window, a.sinks, a.precise, a.new_key == nullptr);
@@ -373,23 +383,24 @@ void lib_attention(const at::Tensor& query, const at::Tensor& codes_k, const std
 
 // ---- steps of the HuggingFace attention forward ----
 
-// q [B, Hq, n, d], k [B, Hkv, n, d] (rows contiguous), cos / sin [B or 1, n, d]
+// q [B, Hq, n, d], k [B, Hkv, n, d], cos / sin [B or 1, n, d]
 // -> the embedded q and k, [B, H, n, d] views of [B, n, H, d] storage
-std::tuple<at::Tensor, at::Tensor> rope(const at::Tensor& q, const at::Tensor& k, const at::Tensor& cos,
-                                        const at::Tensor& sin) {
-  on_device(q, "q");
-  on_device(k, "k");
-  on_device(cos, "cos");
-  on_device(sin, "sin");
+std::tuple<at::Tensor, at::Tensor> rope(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& cos_in,
+                                        const at::Tensor& sin_in) {
+  on_device(q_in, "q");
+  on_device(k_in, "k");
+  on_device(cos_in, "cos");
+  on_device(sin_in, "sin");
+  const c10::DeviceGuard g(q_in.device());
+  const at::Tensor q = rows16(q_in), k = rows16(k_in), cos = rows16(cos_in), sin = rows16(sin_in);
   TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && q.size(0) == k.size(0) && q.size(2) == k.size(2) && q.size(3) == k.size(3),
               "fused_tq: q and k must be [B, H, n, d]");
   const int64_t B = q.size(0), n = q.size(2), d = q.size(3);
   for (const at::Tensor* t : {&cos, &sin})
     TORCH_CHECK(t->dim() == 3 && (t->size(0) == B || t->size(0) == 1) && t->size(1) == n && t->size(2) == d &&
-                    t->stride(2) == 1 && t->scalar_type() == q.scalar_type(),
+                    t->scalar_type() == q.scalar_type(),
                 "fused_tq: cos and sin must be [B or 1, n, d] of q's type");
-  TORCH_CHECK(q.stride(3) == 1 && k.stride(3) == 1 && q.scalar_type() == k.scalar_type(), "fused_tq: rows must be contiguous");
-  const c10::DeviceGuard g(q.device());
+  TORCH_CHECK(q.scalar_type() == k.scalar_type(), "fused_tq: q and k must be of one type");
   at::Tensor qo = at::empty({B, n, q.size(1), d}, q.options()), ko = at::empty({B, n, k.size(1), d}, k.options());
   if (qo.numel() > 0 && ko.numel() > 0)
     check_rc(ftq_rope(q.data_ptr(), qo.data_ptr(), q.stride(0), q.stride(1), q.stride(2), (int)q.size(1), k.data_ptr(),

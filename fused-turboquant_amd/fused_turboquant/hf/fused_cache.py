@@ -377,15 +377,13 @@ def _apply_rotary_pos_emb(q, k, cos, sin):
 def _rope_fused(q, k, cos, sin) -> bool:
     """Whether the rotary embedding of q / k [B, H, n, d] runs as one kernel
     (the same roundings as the torch expression): device tensors of one type,
-    full-width cos / sin, aligned rows, nothing to differentiate."""
+    full-width cos / sin, nothing to differentiate."""
     d = q.shape[-1]
     return (q.is_cuda and q.dtype in (torch.float32, torch.float16, torch.bfloat16) and d % 16 == 0
             and k.dtype == q.dtype and cos.dtype == q.dtype and sin.dtype == q.dtype
             and cos.dim() == 3 and sin.shape == cos.shape and tuple(cos.shape[1:]) == (q.shape[2], d)
             and cos.shape[0] in (1, q.shape[0]) and k.shape[0] == q.shape[0] and k.shape[2:] == q.shape[2:]
-            and not _needs_grad(q, k, cos, sin)
-            and all(t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1])
-                    for t in (q, k, cos, sin)))
+            and not _needs_grad(q, k, cos, sin))
 
 
 def _needs_grad(*tensors) -> bool:

@@ -181,13 +181,6 @@ def paged_decode_attention(query: torch.Tensor, kv_cache: torch.Tensor, block_ta
 LIB_ATTENTION_DIMS = (64, 128, 256)  # head dims of ``lib_attention``
 
 
-def _rows16(t: torch.Tensor) -> torch.Tensor:
-    """``t`` with rows the kernels can read in 16-byte steps (itself where it has them)."""
-    if t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0:
-        return t
-    return t.contiguous()
-
-
 def lib_attention(query: torch.Tensor, lens: torch.Tensor, max_len: int, k_quant: TurboQuantMSE,
                   v_quant: TurboQuantMSE, scale: float, pages: tuple | None = None, flat: tuple | None = None,
                   new_kv: tuple | None = None, window: int | None = None, sinks: int = 0,
@@ -215,12 +208,9 @@ def lib_attention(query: torch.Tensor, lens: torch.Tensor, max_len: int, k_quant
         # ones were exact there (4.4e-4 for 3.4e-4 over 49 + 494 positions, 2.1e-4
         # with precise, whose own output rounding that is)
         precise = new_kv is None or query.dtype != torch.bfloat16
-    q = _rows16(query)
     if out is None:
-        out = torch.empty(B, n, hq, d, dtype=q.dtype, device=q.device).transpose(1, 2)
-    nk = nv = None
-    if new_kv is not None:
-        nk, nv = _rows16(new_kv[0]), _rows16(new_kv[1])
+        out = torch.empty(B, n, hq, d, dtype=query.dtype, device=query.device).transpose(1, 2)
+    nk, nv = new_kv if new_kv is not None else (None, None)
     # beyond the context a window hides nothing and a sink is no position
     most = max(int(max_len), 1)
     window = min(int(window), most) if window else 0
@@ -228,8 +218,8 @@ def lib_attention(query: torch.Tensor, lens: torch.Tensor, max_len: int, k_quant
     kq, vq = k_quant.quantizer, v_quant.quantizer
     codes_k, codes_v, norms_k, norms_v, bt = ((pages[0], None, None, None, pages[1]) if pages is not None else
                                               (flat[0], flat[2], flat[1], flat[3], None))
-    _lib.require_device(q, codes_k, lens, out)
-    _ops.ops().lib_attention(q, codes_k, codes_v, norms_k, norms_v, bt, lens, nk, nv, k_quant.rotation.signs,
+    _lib.require_device(query, codes_k, lens, out)
+    _ops.ops().lib_attention(query, codes_k, codes_v, norms_k, norms_v, bt, lens, nk, nv, k_quant.rotation.signs,
                              v_quant.rotation.signs, kq.levels, vq.levels, k_quant.bits, v_quant.bits, int(max_len),
                              float(scale), window, sinks, bool(precise), out)
     return out

@@ -274,3 +274,40 @@ def test_windows_sinks_and_batches_of_the_torch_form(cuda, d, window, sinks, que
     monkeypatch.setattr(type(cache), "_fused_attention", staticmethod(lambda *a: False))
     want = cache.decode_attention(q, 0, 0.1, sliding_window=window, sink_tokens=sinks).cpu()
     assert got.shape == want.shape and (got - want).norm() <= 1e-5 * want.norm()
+
+
+def _misaligned(t):
+    """The same values, contiguous, at a storage offset of one element."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.reshape(-1)
+    return flat[1:].view(t.shape)
+
+
+def _odd_strides(t):
+    """The same values, with a dimension of size 1 and an odd stride in front, or rows that are not contiguous."""
+    wide = torch.empty(*t.shape[:-1], 2 * t.shape[-1] + 1, dtype=t.dtype, device=t.device)
+    wide[..., 1:] = t.repeat_interleave(2, -1)
+    return wide[..., 1::2]
+
+
+@pytest.mark.parametrize("form", [_misaligned, _odd_strides,
+                                  lambda t: t.contiguous().as_strided(t.shape, (t[0].numel() + 3, *t.stride()[1:]))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_any_alignment_and_stride(cuda, form, dtype):
+    """Queries, new tokens and angles at any storage offset and stride give what aligned ones give."""
+    from fused_turboquant import _ops
+    from fused_turboquant.hf import fused_cache as F
+    d, n = 64, 6
+    cache, g = _cache(cuda, d, 4, 4, 1, 2, (50,), seed=5, dtype=dtype)
+    k, v = (torch.randn(1, 2, n, d, generator=g).to(dtype).to(cuda) for _ in range(2))
+    q = torch.randn(1, 4, n, d, generator=g).to(dtype).to(cuda)
+    cos, sin = (torch.randn(1, n, d, generator=g).to(dtype).to(cuda) for _ in range(2))
+    q1 = q[:, :, 0].contiguous()
+    want = cache.decode_attention(q1, 0, 0.125, sliding_window=20)
+    assert torch.equal(cache.decode_attention(form(q1), 0, 0.125, sliding_window=20), want)
+    cache.store_compressed_kv(k, v, 0)
+    want = cache.chunk_attention(q, k, v, 0, 0.125)
+    assert torch.equal(cache.chunk_attention(form(q), form(k), form(v), 0, 0.125), want)
+    assert F._rope_fused(form(q), form(k), form(cos), form(sin))
+    for a, b in zip(_ops.ops().rope(form(q), form(k), form(cos), form(sin)), _ops.ops().rope(q, k, cos, sin)):
+        assert torch.equal(a, b)

@@ -60,3 +60,26 @@ def test_cpu_tensors_rejected_by_the_package():
     tq = TurboQuantMSE(128, bits=3)
     with pytest.raises(FusedTQError):
         tq.encode(torch.zeros(4, 128))
+
+
+def test_cache_attention_traces_without_data_pointers():
+    """The rotary embedding's route and the library-format attention run under
+    a fake mode without a look at a pointer that is not there."""
+    import warnings
+    from types import SimpleNamespace
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from fused_turboquant import paged as P
+    from fused_turboquant.hf import fused_cache as F
+    ops = _ops()
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("error")
+        def t(*shape, dtype=torch.bfloat16):
+            return torch.empty(*shape, dtype=dtype, device="cuda")
+        q, k, cos = t(2, 8, 5, 128), t(2, 2, 5, 128), t(1, 5, 128)
+        assert F._rope_fused(q, k, cos, cos)
+        assert [x.shape for x in ops.rope(q, k, cos, cos)] == [q.shape, k.shape]
+        quant = SimpleNamespace(bits=4, quantizer=SimpleNamespace(levels=t(16, dtype=torch.float32)),
+                                rotation=SimpleNamespace(signs=t(128, dtype=torch.float32)))
+        pages = (t(8, 2, 1, 2 * 128 * 8 + 64, dtype=torch.uint8), t(2, 4, dtype=torch.int32))
+        out = P.lib_attention(q, t(2, dtype=torch.int32), 40, quant, quant, 0.1, pages=pages, new_kv=(k, k))
+        assert out.shape == q.shape and out.dtype == q.dtype
