@@ -268,8 +268,16 @@ void v1_chunk_attention(const at::Tensor& query, const at::Tensor& kv_cache, con
   TORCH_CHECK_VALUE(past_len >= 0 && past_len <= INT32_MAX && window >= 0 && window <= INT32_MAX &&
                         query.size(0) <= INT32_MAX && block_row.numel() <= INT32_MAX,
                     "fused_tq: past_len / window / token counts out of range");
-  if (centroids.has_value()) contig(*centroids, "centroids");
-  if (rotation.has_value()) contig(*rotation, "rotation");
+  // the kernels read 2^key_bits centroids and a d x d rotation (raw slots and fp8 keys: no centroids)
+  if (centroids.has_value()) {
+    contig(*centroids, "centroids");
+    TORCH_CHECK_VALUE(key_bits < 1 || key_bits > 8 || (v_flags & 4) != 0 || centroids->numel() == ((int64_t)1 << key_bits),
+                      "fused_tq: centroids must have 2^key_bits entries");
+  }
+  if (rotation.has_value()) {
+    contig(*rotation, "rotation");
+    TORCH_CHECK_VALUE(rotation->numel() == query.size(2) * query.size(2), "fused_tq: rotation must be [d, d]");
+  }
   const c10::DeviceGuard g(query.device());
   const int n = (int)query.size(0), hq = (int)query.size(1), d = (int)query.size(2), hkv = (int)kv_cache.size(2);
   if (n == 0) return;

@@ -461,6 +461,10 @@ def v1_chunk_attention(query: torch.Tensor, kv_cache: torch.Tensor, block_row: t
     n, hq, d = query.shape
     if key_bits != RAW_BITS:
         _check_bits(d, key_bits, value_bits, key_fp8)
+        if kv_cache.shape[3] < slot_bytes(d, key_bits, value_bits, key_fp8):
+            raise ValueError("kv_cache slot is smaller than the slot bytes for these bits")
+        if not key_fp8 and (centroids is None or centroids.dtype != torch.float32 or centroids.numel() != 1 << key_bits):
+            raise ValueError("centroids must be float32 with 2^key_bits entries")
     if block_row.dtype != torch.int32 or block_row.dim() != 1:
         raise ValueError("block_row must be int32 [max_blocks]")
     tensors = [query, kv_cache, block_row] + ([centroids] if centroids is not None else [])

@@ -206,3 +206,26 @@ def test_an_infinite_raw_value_stays_in_the_rows_that_attend_it(cuda, d, past):
     got = _chunk(None, q, cache, row, past, RAW, RAW, False)
     assert torch.equal(got[:at], want[:at])
     assert torch.isnan(got[at:, :, [5, d - 1]]).all()
+
+
+def test_chunk_rejects_tables_of_another_width():
+    """Refused before a device is asked for: the kernel reads 2^key_bits centroids."""
+    from fused_turboquant import v1 as V1
+    q, row = torch.zeros(16, 4, 64), torch.zeros(4, dtype=torch.int32)
+    cache = torch.zeros(4, 16, 1, V1.slot_bytes(64, 4, 4), dtype=torch.uint8)
+    for cent in (None, torch.zeros(8), torch.zeros(32), torch.zeros(16, dtype=torch.float64)):
+        with pytest.raises(ValueError, match="centroids"):
+            V1.v1_chunk_attention(q, cache, row, 8, cent, 4, 4, 0.125)
+    with pytest.raises(ValueError, match="slot"):
+        V1.v1_chunk_attention(q, cache[..., :32], row, 8, torch.zeros(16), 4, 4, 0.125)
+
+
+@pytest.mark.gpu
+def test_chunk_operator_rejects_tables_of_another_width(cuda):
+    """The operator's own check: an error from the host, no launch."""
+    from fused_turboquant import _ops
+    layer, cache, row = _case(cuda, 64, 4, 4, 1, 40, True, 16, seed=8)
+    q = torch.zeros(20, 4, 64, device=cuda)
+    for cent, rot in ((layer.centroids[:8].contiguous(), None), (layer.centroids, torch.zeros(32, 64, device=cuda))):
+        with pytest.raises(ValueError):
+            _ops.ops().v1_chunk_attention(q, cache, row, 20, cent, 4, 4, 0.125, 1, 0, torch.empty_like(q), rot)
