@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void chunk_gather_lib_kernel(const LibSource s
   __shared__ int tpos[32];  // the token's position, or -1 (hidden)
   __shared__ int tnew[32];  // its index among the new tokens, or -1
   const int tile = blockIdx.x, unit = blockIdx.y, b = unit / hkv, kvh = unit - b * hkv, tid = threadIdx.x;
-  const int len = s.lens[b], past = len - s.n_new;
+  const int len = s.paged ? s.lens[b] : min(s.lens[b], s.cap), past = len - s.n_new;  // flat rows end at the capacity
   const int v0 = seg0 + tile * 32;
   const int lo = s.window > 0 ? max(0, len - s.window) : 0;
   const int kd = D * s.kb / 32, vd = D * s.vb / 32, cw = D * s.vb / 128;  // dwords: codes of a token, a V lane chunk

@@ -311,3 +311,15 @@ def test_any_alignment_and_stride(cuda, form, dtype):
     assert F._rope_fused(form(q), form(k), form(cos), form(sin))
     for a, b in zip(_ops.ops().rope(form(q), form(k), form(cos), form(sin)), _ops.ops().rope(q, k, cos, sin)):
         assert torch.equal(a, b)
+
+
+def test_flat_rows_end_at_the_capacity(cuda):
+    """A length beyond the rows' capacity counts as the capacity."""
+    cache, g = _cache(cuda, 64, 4, 4, 2, 2, (100, 100), seed=6)
+    cap = cache._pages[0].cap
+    q = torch.randn(2, 4, 1, 64, generator=g).to(cuda)
+    lens = torch.tensor([cap, 70], dtype=torch.int32, device=cuda)
+    want = _lib(cache, q, window=60, lens=lens, max_len=cap)
+    lens[0] = cap + 40
+    got = _lib(cache, q, window=60, lens=lens, max_len=cap)
+    assert torch.equal(got, want)
