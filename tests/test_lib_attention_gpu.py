@@ -323,3 +323,52 @@ def test_flat_rows_end_at_the_capacity(cuda):
     lens[0] = cap + 40
     got = _lib(cache, q, window=60, lens=lens, max_len=cap)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("d,dtype", [(64, torch.float32), (128, torch.bfloat16), (256, torch.float16)])
+def test_multi_token_step_lengths_strides_and_streams(cuda, d, dtype):
+    """Sequences of different lengths, queries and new tokens as the transposed
+    views a projection gives, on a stream other than the default one."""
+    B, hkv, G, n, lens = 2, 2, 3, 25, (90, 33)
+    cache, g = _cache(cuda, d, 4, 3, B, hkv, lens, seed=d + 7, dtype=dtype)
+    kd, vd = (_decoded(cache, w, B, hkv, d) for w in "kv")
+    k, v = (torch.randn(B, n, hkv, d, generator=g).to(dtype).transpose(1, 2) for _ in range(2))
+    q = torch.randn(B, n, hkv * G, d, generator=g).to(dtype).transpose(1, 2)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        qc, kc, vc = (t.transpose(1, 2).to(cuda).transpose(1, 2) for t in (q, k, v))
+        assert not (qc.is_contiguous() or kc.is_contiguous())
+        cache.store_compressed_kv(kc, vc, 0)
+        got = cache.chunk_attention(qc, kc, vc, 0, 1 / math.sqrt(d), sliding_window=60).float().cpu().numpy()
+    for b, past in enumerate(lens):
+        row, col = past + np.arange(n)[:, None], np.arange(past + n)[None]
+        ok = (col <= row) & (col > row - 60)
+        for h in range(hkv * G):
+            kk = np.concatenate([kd[b, h // G, :past], k[b, h // G].double().numpy()])
+            vv = np.concatenate([vd[b, h // G, :past], v[b, h // G].double().numpy()])
+            want = _attend(q[b, h].double().numpy(), kk, vv, 1 / math.sqrt(d), ok)
+            tol = {torch.float32: 1e-5, torch.float16: 1e-5 + 2.0 ** -11, torch.bfloat16: 1e-3 + 2.0 ** -9}[dtype]
+            assert _rel(got[b, h], want) < tol, (b, h)
+
+
+def test_several_segments(cuda):
+    """A context whose dequantised fragments exceed one workspace segment (192
+    MiB: 5952 positions of 64 kv heads at d = 64), in a decode step and in a
+    multi-token step."""
+    d, B, hkv, past, n = 64, 4, 16, 6100, 6
+    cache, g = _cache(cuda, d, 2, 3, B, hkv, (past,) * B, seed=9)
+    kd, vd = (_decoded(cache, w, B, hkv, d) for w in "kv")
+    q = torch.randn(B, hkv, n, d, generator=g)
+    got = cache.decode_attention(q[:, :, 0].to(cuda), 0, 0.125).cpu().numpy()
+    every = np.ones((1, past), bool)
+    want = np.stack([[_attend(q[b, h, :1].double().numpy(), kd[b, h, :past], vd[b, h, :past], 0.125, every)[0]
+                      for h in range(hkv)] for b in range(B)])
+    assert _rel(got, want) < 1e-5
+    k, v = (torch.randn(B, hkv, n, d, generator=g) for _ in range(2))
+    cache.store_compressed_kv(k.to(cuda), v.to(cuda), 0)
+    got = cache.chunk_attention(q.to(cuda), k.to(cuda), v.to(cuda), 0, 0.125).cpu().numpy()
+    ok = np.arange(past + n)[None] <= past + np.arange(n)[:, None]
+    want = np.stack([[_attend(q[b, h].double().numpy(), np.concatenate([kd[b, h, :past], k[b, h].double().numpy()]),
+                              np.concatenate([vd[b, h, :past], v[b, h].double().numpy()]), 0.125, ok)
+                      for h in range(hkv)] for b in range(B)])
+    assert _rel(got, want) < 1e-5
